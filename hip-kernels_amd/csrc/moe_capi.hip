@@ -654,6 +654,7 @@ static int layer_experts(gptoss_moe_layer* L, const Scratch& S, const uint16_t* 
     g.limit = c.swiglu_limit;
     g.queue = S.gqueue;
     g.num_cus = L->num_cus;
+    g.x_rows = T;
     g.timer = pf.timer(1);
     if (c.prefill_block_scaled) {  // the tokens as e4m3 parts, then block-scaled products
       const KernelTimer t1 = pf.timer(1);
@@ -668,6 +669,7 @@ static int layer_experts(gptoss_moe_layer* L, const Scratch& S, const uint16_t* 
     }
     HIP_TRY(launch_grouped_mxfp4(g, s), "grouped gate_up launch");
     g.x = S.act;
+    g.x_rows = g.rows;
     g.row_index = nullptr;
     if (c.prefill_block_scaled) {
       g.xq = S.aq;
@@ -1112,6 +1114,10 @@ int gptoss_moe_grouped_mxfp4_gemm(const uint16_t* x, const int32_t* row_index, c
   g.gated = swiglu != 0;
   g.alpha = alpha;
   g.limit = limit;
+  g.x_rows = row_index == nullptr ? rows : 0;  // a gather's row numbers are not known here
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev), "hipGetDevice");
+  HIP_TRY(hipDeviceGetAttribute(&g.num_cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
   HIP_TRY(launch_grouped_mxfp4(g, static_cast<hipStream_t>(stream)), "grouped gemm launch");
   return ok();
 }

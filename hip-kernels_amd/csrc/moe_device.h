@@ -164,6 +164,7 @@ __device__ __forceinline__ bool has_special_code(uint32_t v, uint32_t mask) {
   return (((x - 0x01010101u) & ~x & 0x80808080u) | ((y - 0x01010101u) & ~y & 0x80808080u)) != 0u;
 }
 
+typedef uint32_t gx_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t gx_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 gx_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 gx_bf16x2 __attribute__((ext_vector_type(2)));

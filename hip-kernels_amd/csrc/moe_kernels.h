@@ -212,7 +212,8 @@ struct GroupedArgs {
   int gated;
   float alpha, limit;
   int32_t* queue;  // null, or grouped_queue_ints() zeroed ints (persistent grid; left zeroed)
-  int num_cus;     // with a queue: compute units of the device
+  int num_cus;     // with a queue, and for the mid stream: compute units of the device
+  int x_rows;      // rows of x when known, else 0 (the mid stream needs it)
   KernelTimer timer;
   // Block-scaled variant (v_mfma_scale_f32_16x16x128_f8f6f4, fp4 weights x
   // fp8 activations): xq / xqs non-null select it.  xq, xqs: the rows of x
@@ -230,6 +231,12 @@ struct GroupedArgs {
 constexpr int grouped_queue_ints() { return 9 * 32; }
 bool grouped_supported(int N, int K, int E);
 hipError_t launch_grouped_mxfp4(const GroupedArgs& a, hipStream_t s);
+// The same product streamed for a few tokens per expert (moe_midstream.hip),
+// which launch_grouped_mxfp4 selects where it pays and is supported (chunk
+// table, 32-bit buffer offsets, the rows of x known).
+bool mid_stream_pays(const GroupedArgs& a);
+bool mid_stream_supported(const GroupedArgs& a);
+hipError_t launch_mid_stream(const GroupedArgs& a, hipStream_t s);
 
 // Activations for the block-scaled products: every 32-element block of a bf16
 // row becomes two e4m3 parts with one power-of-two scale s = 2^(e - 7), e the

@@ -1065,6 +1065,7 @@ bool grouped_supported(int N, int K, int E) {
 hipError_t launch_grouped_mxfp4(const GroupedArgs& a, hipStream_t s) {
   if (a.rows <= 0) return hipSuccess;
   if (!grouped_supported(a.N, a.K, a.E)) return hipErrorInvalidValue;
+  if (mid_stream_pays(a) && mid_stream_supported(a)) return launch_mid_stream(a, s);
   GroupedParams p{};
   p.x = a.x;
   p.row_index = a.row_index;
