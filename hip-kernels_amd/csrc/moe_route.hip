@@ -42,7 +42,11 @@ namespace {
 
 constexpr int kRouteThreads = 256;
 constexpr int kPlanThreads = 1024;
-constexpr int kTopkPlanMaxT = 256;  // tokens of the single-work-group top-k + plan
+// Tokens of the single-work-group top-k + plan.  Above, its waves select
+// several tokens each in turn and the top-k of its own launch over the chip,
+// followed by plan_kernel, is ahead (GPT-OSS-120B: 31-35 us at 200 tokens
+// against 4.9 + 4.8).
+constexpr int kTopkPlanMaxT = 64;
 
 // Dispatch plan over the T*k slots of `idx` with NT threads: counts,
 // exclusive offsets, a gather map that is stable in slot order (the counting
@@ -1024,7 +1028,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t* idx, 
 hipError_t launch_plan_kernel(const int32_t* idx, int T, int k, int E, PlanBufs plan, hipStream_t s,
                               const KernelTimer& timer) {
   const int S = T * k;
-  if (plan.chunk != nullptr && S > kPlanChunkSlots) {  // three launches over the device
+  // Three launches over the device above kPlanOneGroupSlots: plan_kernel takes
+  // 4.3 us at 512 slots, 6.6 at 2048, 9.6 at 4096, 12.5 at 6144 and 15.4 at
+  // 8192; the three take 11.3 us at 4004 slots and the gaps between them.
+  constexpr int kPlanOneGroupSlots = 4096;
+  if (plan.chunk != nullptr && S > kPlanOneGroupSlots) {
     const int NB = (S + kPlanChunkSlots - 1) / kPlanChunkSlots;
     gx_launch(plan_count_kernel, dim3(NB), dim3(kChunkThreads), 0, s, KernelTimer{timer.start, nullptr}, idx, S, E,
               plan.chunk);
