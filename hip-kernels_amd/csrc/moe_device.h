@@ -169,18 +169,15 @@ typedef uint32_t gx_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 gx_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 gx_bf16x2 __attribute__((ext_vector_type(2)));
 
-// Row r's 16 bytes of one tiled MXFP4 block (layout in moe_kernels.h), given
-// p = &block[tiled_dword(r, 0)]: dword g is slot 16 g + r % 16, 64 dwords
-// after dword g - 1.  Nontemporal: streamed weights are read once.
-__device__ __forceinline__ gx_u32x4 load_row_block_nt(const uint32_t* p) {
-  gx_u32x4 v;
-  v[0] = __builtin_nontemporal_load(p);
-  v[1] = __builtin_nontemporal_load(p + 64);
-  v[2] = __builtin_nontemporal_load(p + 128);
-  v[3] = __builtin_nontemporal_load(p + 192);
-  return v;
+// The lane's 16-byte slot of one tiled MXFP4 block (p = its address).
+// Nontemporal: streamed weights are read once.
+__device__ __forceinline__ gx_u32x4 load_slot_nt(const uint32_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const gx_u32x4*>(p));
 }
 
+// Row r's 16 bytes of one tiled MXFP4 block (layout in moe_kernels.h), given
+// p = &block[tiled_dword(r, 0)]: dword g is slot 16 g + r % 16, 64 dwords
+// after dword g - 1.
 __device__ __forceinline__ gx_u32x4 load_row_block(const uint32_t* p) {
   gx_u32x4 v;
   v[0] = p[0];
@@ -188,6 +185,18 @@ __device__ __forceinline__ gx_u32x4 load_row_block(const uint32_t* p) {
   v[2] = p[128];
   v[3] = p[192];
   return v;
+}
+
+// The lane's 16-byte slot of a tiled block (slot 16 a + j: dword i = bytes
+// 4a..4a+3 of row 16 i + j) -> row `lane`'s own 16 bytes in order: a 4 x 4
+// transpose of dwords over the wave's four rows of 16 lanes.  One coalesced
+// 16-byte load and four swaps in place of load_row_block's four dword loads.
+__device__ __forceinline__ gx_u32x4 slot_to_row(const gx_u32x4& v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return gx_u32x4{c[0], c[1], d[0], d[1]};
 }
 
 // Eight e2m1 values (one dword, low nibble first) times the e8m0 scale as

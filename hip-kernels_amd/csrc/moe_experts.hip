@@ -212,7 +212,7 @@ void expert_stream_kernel(StreamParams a) {
     const int pp = s.valid ? p : 0;
     const size_t eoff = s.valid ? static_cast<size_t>(s.e) * g.nib_bytes : 0;
     return reinterpret_cast<const uint32_t*>(a.wn + eoff + static_cast<size_t>(t) * tile_bytes) +
-           static_cast<size_t>(pp) * bpp * 256 + tiled_dword(lane, 0);
+           static_cast<size_t>(pp) * bpp * 256 + 4 * lane;
   };
   auto ssrc = [&](const Step& s, int r) -> const uint32_t* {
     const int t = s.valid ? min(s.tp * R + r, ntiles - 1) : 0;
@@ -294,7 +294,7 @@ void expert_stream_kernel(StreamParams a) {
       const uint32_t* src = wsrc(cur, r, stride);
 #pragma unroll
       for (int i = 0; i < kD; ++i)
-        if (BPP || i < bpp) ring[r][i] = load_row_block_nt(src + static_cast<size_t>(i) * stride);
+        if (BPP || i < bpp) ring[r][i] = load_slot_nt(src + static_cast<size_t>(i) * stride);
     }
   }
   if (static_cast<int>(threadIdx.x) < kMaxExperts)
@@ -405,12 +405,15 @@ void expert_stream_kernel(StreamParams a) {
           spc[r] = (code - 1u) >= 254u;
           cs[r] = spc[r] ? 1.0f : scf[r];
         }
+        u32x4 wr[R];  // the row's 16 bytes
+#pragma unroll
+        for (int r = 0; r < R; ++r) wr[r] = slot_to_row(ring[r][i % kD]);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           float wf[R][8];
 #pragma unroll
           for (int r = 0; r < R; ++r) {
-            decode8_regular(ring[r][i % kD][d], cs[r], wf[r]);
+            decode8_regular(wr[r][d], cs[r], wf[r]);
             if (wave_sp) {
               // codes 0 and 255: exact e2m1 values times the IEEE scale
 #pragma unroll
@@ -439,10 +442,10 @@ void expert_stream_kernel(StreamParams a) {
       for (int r = 0; r < R; ++r) {
         if (ni < kLoop) {
           if (BPP || ni < bpp)
-            ring[r][i % kD] = load_row_block_nt(csrc[r] + static_cast<size_t>(ni) * cstride[r]);
+            ring[r][i % kD] = load_slot_nt(csrc[r] + static_cast<size_t>(ni) * cstride[r]);
         } else {
           if (BPP || ni - kLoop < bpp)
-            ring[r][i % kD] = load_row_block_nt(nsrc[r] + static_cast<size_t>(ni - kLoop) * nstride[r]);
+            ring[r][i % kD] = load_slot_nt(nsrc[r] + static_cast<size_t>(ni - kLoop) * nstride[r]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);

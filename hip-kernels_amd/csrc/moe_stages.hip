@@ -20,47 +20,106 @@ namespace gxmoe {
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-constexpr int kRows = 8;  // token rows per work-group of the dense GEMV
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Dense MXFP4 GEMV: grid (N/64 tiles, ceil(M/8)), 64*P threads.  Lane = row
-// of the tile, wave = K-part; same canonical dot as the fused expert kernels.
+// Dense MXFP4 GEMV: grid (N/64 tiles, ceil(M / TC)), 64 parts threads.  Lane =
+// row of the tile, wave = K-part; same canonical dot as the fused expert
+// kernels: one ascending fmaf chain per (row, token) over the part, the part
+// sums added in part order, + bias.
+//
+// Bound by the chains (a part is 480 dependent fmaf at K = 2880) and the
+// issue of its loads.  A block of weights is one coalesced 16-byte load per
+// lane, put in row order by four lane swaps (four dword loads per block, each
+// over the same KiB, and a byte load per scale made a second work-group on a
+// CU double its time).  The token values are the same for every lane, so they
+// come through the scalar cache into scalar registers, a block of a row in one
+// 64-byte load, and each fmaf takes one as its scalar operand (as LDS
+// broadcasts, 16 bytes per four fmaf, they ran at the LDS rate).  The block
+// loop is kept rolled: unrolled over the part it waits for instructions.
+// Measured, N = 5760, K = 2880, M = 1 / 5 / 16 / 64: 20.5 / 48 / 70 / 115 us
+// before, 8.1 / 13.1 / 21 / 62 now.
+template <int TC, bool kAligned>
 __global__ __launch_bounds__(kTileRows * kMaxParts) void dense_gemv_kernel(
     const uint16_t* __restrict__ x, int M, const uint8_t* __restrict__ wn, const uint8_t* __restrict__ ws,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, TiledGeom g) {
-  __shared__ float s_part[kMaxParts][kRows][kTileRows];
+  constexpr int kD = 4;  // weight blocks in flight (a dword of scale codes)
+  __shared__ float s_part[kMaxParts][TC][kTileRows];
   const int tile = blockIdx.x;
-  const int m0 = blockIdx.y * kRows;
-  const int mc = min(kRows, M - m0);
+  const int m0 = blockIdx.y * TC;
+  const int mc = min(TC, M - m0);
   const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int K = g.K;
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(wn + static_cast<size_t>(tile) * g.nb * 1024) +
-                        static_cast<size_t>(p) * g.bpp * 256 + tiled_dword(lane, 0);
+  const int K = g.K, bpp = g.bpp;
+  const u32x4* src =
+      reinterpret_cast<const u32x4*>(wn + (static_cast<size_t>(tile) * g.nb + static_cast<size_t>(p) * bpp) * 1024) + lane;
   const uint8_t* sc = ws + (static_cast<size_t>(tile) * g.parts + p) * kTileRows * g.spad +
                       static_cast<size_t>(lane) * g.spad;
-  float acc[kRows];
+  uint32_t codes[4];  // the part's scale codes, at most 16
+  if (kAligned) {
 #pragma unroll
-  for (int m = 0; m < kRows; ++m) acc[m] = 0.0f;
-  for (int i = 0; i < g.bpp; ++i) {
-    const u32x4 blk = load_row_block(src + static_cast<size_t>(i) * 256);
-    const uint32_t code = sc[i];
-    const int kb = (p * g.bpp + i) * 32;
+    for (int q = 0; q < 4; ++q) codes[q] = reinterpret_cast<const uint32_t*>(sc)[min(q, (g.spad >> 2) - 1)];
+  } else {
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      float wf[8];
-      decode8(blk[d], code, wf);
+    for (int q = 0; q < 4; ++q) {
+      codes[q] = 0;
 #pragma unroll
-      for (int m = 0; m < kRows; ++m) {
-        if (m < mc) {
-          const uint16_t* xr = x + static_cast<size_t>(m0 + m) * K + kb + d * 8;
+      for (int r = 0; r < 4; ++r) codes[q] |= static_cast<uint32_t>(sc[min(4 * q + r, g.spad - 1)]) << (8 * r);
+    }
+  }
+  u32x4 wv[kD];
 #pragma unroll
-          for (int c = 0; c < 8; ++c) acc[m] = __builtin_fmaf(bf16_to_f32(xr[c]), wf[c], acc[m]);
+  for (int u = 0; u < kD; ++u) wv[u] = src[static_cast<size_t>(min(u, bpp - 1)) * 64];
+  const uint16_t* xr[TC];  // rows past M: the last row, their sums are not stored
+#pragma unroll
+  for (int m = 0; m < TC; ++m) xr[m] = x + static_cast<size_t>(m0 + min(m, mc - 1)) * K + p * bpp * 32;
+  float acc[TC];
+#pragma unroll
+  for (int m = 0; m < TC; ++m) acc[m] = 0.0f;
+#pragma clang loop unroll(disable)
+  for (int i0 = 0; i0 < bpp; i0 += kD) {
+#pragma unroll
+    for (int u = 0; u < kD; ++u) {
+      const int i = i0 + u;
+      if (i < bpp) {
+        float wf[32];
+        const uint32_t code = (codes[0] >> (8 * (i & 3))) & 0xffu;
+        const bool sp = (code - 1u) >= 254u;  // a scale code 0 or 255
+        const float scale = e8m0_to_f32(code);
+        const u32x4 wr = slot_to_row(wv[u]);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) decode8_regular(wr[d], sp ? 1.0f : scale, wf + 8 * d);
+        if (__ballot(sp) != 0ull) {
+#pragma unroll
+          for (int c = 0; c < 32; ++c) wf[c] = sp ? wf[c] * scale : wf[c];
+        }
+        wv[u] = src[static_cast<size_t>(min(i + kD, bpp - 1)) * 64];
+        if constexpr (kAligned) {
+          uint32_t xv[TC][16];
+#pragma unroll
+          for (int m = 0; m < TC; ++m)
+#pragma unroll
+            for (int c = 0; c < 16; ++c) xv[m][c] = reinterpret_cast<const uint32_t*>(xr[m] + 32 * i)[c];
+#pragma unroll
+          for (int c = 0; c < 16; ++c) {  // the rows' chains side by side
+#pragma unroll
+            for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(__uint_as_float(xv[m][c] << 16), wf[2 * c], acc[m]);
+#pragma unroll
+            for (int m = 0; m < TC; ++m)
+              acc[m] = __builtin_fmaf(__uint_as_float(xv[m][c] & 0xffff0000u), wf[2 * c + 1], acc[m]);
+          }
+        } else {
+#pragma unroll
+          for (int c = 0; c < 32; ++c)
+#pragma unroll
+            for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(bf16_to_f32(xr[m][32 * i + c]), wf[c], acc[m]);
         }
       }
     }
+    codes[0] = codes[1];
+    codes[1] = codes[2];
+    codes[2] = codes[3];
   }
 #pragma unroll
-  for (int m = 0; m < kRows; ++m)
-    if (m < mc) s_part[p][m][lane] = acc[m];
+  for (int m = 0; m < TC; ++m) s_part[p][m][lane] = acc[m];
   __syncthreads();
   for (int q = threadIdx.x; q < mc * kTileRows; q += blockDim.x) {
     const int m = q >> 6, r = q & 63;
@@ -243,8 +302,28 @@ hipError_t launch_dense_gemv(const uint16_t* x, int M, const uint8_t* wn, const 
                              uint16_t* y, int N, int K, hipStream_t s) {
   if (M <= 0) return hipSuccess;
   const TiledGeom g = tiled_geom(N, K);
-  hipLaunchKernelGGL(dense_gemv_kernel, dim3(N / kTileRows, (M + kRows - 1) / kRows), dim3(kTileRows * g.parts), 0,
-                     s, x, M, wn, ws, bias, y, g);
+  // Token rows per work-group, by the work-groups that one each would make
+  // (N = 5760: 8 rows 15.6 / 17.6 / 15.0 us for 1 / 2 / 4 each, 11 rows 17.4 /
+  // 19.6 / 24, 24 rows 34 / 27 / 30, 64 rows 73 / 59 / 62; N = 2880, K = 1536:
+  // 16 rows 8.9 / 9.9 / 9.4, 32 rows 13.9 / 11.9 / 14.9, 64 rows 24 / 19 / 18).
+  const int tiles = N / kTileRows;
+  const long groups = static_cast<long>(tiles) * M;
+  const int tc = groups <= 1024 ? 1 : groups <= 2560 ? 2 : 4;
+  // x is only 2-byte aligned by contract, the scales not at all
+  const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(ws)) & 3u) == 0;
+#define GX_GEMV(TC_, A_)                                                                                            \
+  hipLaunchKernelGGL((dense_gemv_kernel<TC_, A_>), dim3(tiles, (M + TC_ - 1) / TC_), dim3(kTileRows* g.parts), 0, s, \
+                     x, M, wn, ws, bias, y, g)
+#define GX_GEMV_L(TC_)               \
+  do {                               \
+    if (aligned) GX_GEMV(TC_, true); \
+    else GX_GEMV(TC_, false);        \
+  } while (0)
+  if (tc == 1) GX_GEMV_L(1);
+  else if (tc == 2) GX_GEMV_L(2);
+  else GX_GEMV_L(4);
+#undef GX_GEMV_L
+#undef GX_GEMV
   return hipGetLastError();
 }
 

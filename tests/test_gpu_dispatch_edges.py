@@ -1,0 +1,87 @@
+"""Sizes at the edges of the dispatch rules, against the oracle or a plain
+restatement: the dense GEMV's rows per work-group, unaligned inputs and scale
+codes 0 and 255; the layer's routing plan around the sizes where its launches
+change."""
+import numpy as np
+import pytest
+import torch
+
+import gptoss_moe as g
+import moe_data
+import moe_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a):
+    if a.dtype == np.uint16:
+        return torch.from_numpy(a.view(np.int16)).view(torch.bfloat16).cuda()
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _bits(t):
+    return t.cpu().view(torch.int16).numpy().view(np.uint16)
+
+
+# one, two and four rows per work-group (tiles x M up to 1024, 2560, above);
+# 1, 2, 5, 15 and 16 blocks per K-part; x on 16 or 2 bytes
+@pytest.mark.parametrize("N,K", [(64, 32), (128, 320), (192, 960), (2880, 2880), (512, 2048)])
+@pytest.mark.parametrize("M", [1, 7, 23, 57, 130])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemv_rows(N, K, M, shift):
+    rng = np.random.default_rng([N, K, M])
+    x = moe_data.bf16(rng.normal(0, 1, (M, K)))
+    packed = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    scales = rng.integers(119, 124, (N, K // 32), dtype=np.uint8)
+    scales[5, -1], scales[N - 1, 0] = 0, 255
+    packed[N - 1, :16] = 0x22  # times +inf: no 0 * inf
+    bias = moe_data.bf16(rng.normal(0, 0.5, N))
+    nib, sc = g.pack_tiled(_dev(packed), _dev(scales), N, K)
+    buf = torch.zeros(M * K + 8, dtype=torch.bfloat16, device="cuda")
+    xs = buf[shift:shift + M * K].view(M, K)
+    xs.copy_(_dev(x))
+    y = _bits(g.mxfp4_gemv(xs, nib, sc, _dev(bias), N, K))
+    ref = orc.mxfp4_gemv(x, packed, scales, bias, N, K)
+    nan = np.isnan(orc.bf16_to_f32(ref))
+    assert np.array_equal(np.isnan(orc.bf16_to_f32(y)), nan)
+    assert np.array_equal(y[~nan], ref[~nan])
+
+
+# top-k and plan in one launch up to 64 tokens, plan in one work-group up to
+# 4096 slots, over the chip above
+@pytest.mark.parametrize("E,k", [(30, 4), (64, 8), (128, 4)])
+@pytest.mark.parametrize("T", [63, 64, 65, 255, 257, 512, 513, 1024, 1025])
+def test_layer_plan(E, k, T):
+    H = I = 128
+    w = moe_data.make_layer(3, E, H, I, bias="random")
+    x, res = moe_data.make_tokens(T, T, H)
+    cfg = g.default_config(E, T)
+    cfg.hidden_size, cfg.intermediate_size, cfg.top_k = H, I, k
+    t = {n: _dev(v) for n, v in w.items()}
+    layer = g.MoELayer().init(cfg, 0, t["router_w"], t["router_b"], t["w1_bias"], t["w2_bias"],
+                              mlp1=([t["w1_packed"][e] for e in range(E)], [t["w1_scales"][e] for e in range(E)]),
+                              mlp2=([t["w2_packed"][e] for e in range(E)], [t["w2_scales"][e] for e in range(E)]))
+    layer.forward_prenormed(_dev(x), _dev(res))
+    torch.cuda.synchronize()
+    tr = layer.trace()
+
+    def read(p, n, dt=torch.int32):
+        return g.copy_device_to_tensor(p, n * 4, dt).cpu().numpy()
+
+    S = T * k
+    idx = read(tr.expert_indices, S).reshape(T, k)
+    logits = g.copy_device_to_tensor(tr.logits, T * E * 2, torch.bfloat16).view(T, E)
+    ri, rw = g.topk_softmax(logits, k)
+    assert np.array_equal(idx, ri.cpu().numpy())
+    assert np.array_equal(read(tr.expert_weights, S), rw.cpu().view(torch.int32).numpy().ravel())
+    order = np.argsort(idx.ravel(), kind="stable")
+    counts = np.bincount(idx.ravel(), minlength=E)
+    gmap = np.empty(S, np.int32)
+    gmap[order] = np.arange(S)
+    act = np.flatnonzero(counts)
+    assert np.array_equal(read(tr.expert_counts, E), counts)
+    assert np.array_equal(read(tr.expert_offsets, E + 1), np.concatenate([[0], np.cumsum(counts)]))
+    assert np.array_equal(read(tr.gather_map, S), gmap)
+    assert np.array_equal(read(tr.perm_token, S), order // k)
+    assert read(tr.n_active, 1)[0] == act.size and np.array_equal(read(tr.active_experts, E)[:act.size], act)
+    layer.destroy()
