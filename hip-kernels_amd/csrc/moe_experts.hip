@@ -66,14 +66,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Per work-group LDS: each wave's staged activations (fp32, TC token rows of
 // its K-part, which after the wave's dot hold its part sums), the packed
 // header of every active-expert task record ({expert | count << 8, offset})
-// and, for small batches, the slot -> token map.  Kept under a third of the
-// CU's 160 KiB, so the compiler does not budget for fewer resident waves
-// (which also sets the VGPR allocation it reports to the dispatcher).
-template <int PK, int TC, int kTok>
+// and the running count of the chunks past each expert's first.  Kept under a
+// third of the CU's 160 KiB, so the compiler does not budget for fewer
+// resident waves (which also sets the VGPR allocation it reports to the
+// dispatcher).
+template <int PK, int TC>
 struct StreamSmem {
   float x[kMaxParts][TC][PK];
   int2 hdr[kMaxExperts];
-  int32_t tok[kTok];
+  int32_t more[kMaxExperts];  // chunks c >= 1 of records 0 .. i
 };
 
 // Activations of one token chunk for one wave's K-part: lane l moves 16-byte
@@ -129,7 +130,6 @@ struct StreamParams {
   const int32_t* tasks;       // [max_active][kTaskInts] task records
   const int32_t* n_active;    // [1]
   const int32_t* perm_token;  // [S] token of each permuted slot (gate_up only)
-  int slots;                  // S = T * top_k
   uint16_t* out;              // gate_up: SwiGLU activations [S][N/2]; down: expert outputs [S][N]
   uint16_t* gate_up;          // [S][N] bf16 trace or null (gate_up only)
   int max_active;
@@ -138,15 +138,19 @@ struct StreamParams {
 };
 
 // One step of a work-group's stream: tile group tp (R tiles) of the j-th
-// active expert, token chunk c.
+// active expert, token chunk c; q is its place in the list of steps.
 struct Step {
-  int valid, j, tp, c, e, off, M;
+  int valid, q, j, tp, c, e, off, M;
 };
 
-// The persistent expert stream.  Work-group b takes the items (j, tp) =
-// b, b + G, ... of the n_active x ceil(tiles/R) item list (G = grid size) and
-// each item's token chunks in order; each step applies the R tiles' weights
-// to up to TC tokens.  Lane l of wave p owns row l of each tile and runs, per
+// The persistent expert stream.  A step applies R tiles' weights of an active
+// expert to a chunk of up to TC of its tokens; work-group b takes the steps
+// b, b + G, ... (G = grid size) of the list that holds every expert's first
+// chunk, tile group by tile group, and then the experts' further chunks
+// likewise.  (A chunk reads its weights again either way, so a work-group that
+// kept all chunks of its tiles only made the busiest expert the longest wait:
+// 24 tokens, 32 experts, both launches: Zipf routing 380 us so and 170 as
+// single steps, uniform routing 192 and 166.)  Lane l of wave p owns row l of each tile and runs, per
 // token, one ascending fmaf chain over K-part p (the canonical dot); the part
 // sums are added in part order across the work-group, which then adds the
 // bias and emits (gate_up: bf16 gate/up values, clamped SwiGLU on lane pairs,
@@ -158,12 +162,12 @@ struct Step {
 // activation pieces and token ids are issued during the current step, so a
 // wave's loads never stop between steps; loads for a step that does not
 // exist read a fixed valid location (static wait counts, no stray traffic).
-template <int BPP, int R, int TC, int D, bool kGated, int kTok>
-__global__ __launch_bounds__(kTileRows * kMaxParts) __attribute__((amdgpu_waves_per_eu(4)))
+template <int BPP, int R, int TC, int D, bool kGated>
+__global__ __launch_bounds__(kTileRows * kMaxParts) __attribute__((amdgpu_waves_per_eu(R == 1 ? 5 : 4)))
 void expert_stream_kernel(StreamParams a) {
   constexpr int PK = PartLen<BPP, R>::kValue;
   static_assert(TC * R * kTileRows <= TC * PK, "part sums fit the staged rows");
-  __shared__ __attribute__((aligned(16))) StreamSmem<PK, TC, kTok> sm;
+  __shared__ __attribute__((aligned(16))) StreamSmem<PK, TC> sm;
   constexpr int kLoop = BPP ? BPP : kMaxBpp;
   constexpr int kD = D < kLoop ? D : kLoop;
   static_assert(kLoop % kD == 0, "ring depth must divide the part length");
@@ -178,30 +182,82 @@ void expert_stream_kernel(StreamParams a) {
   const int G = gridDim.x;
   const size_t tile_bytes = static_cast<size_t>(g.nb) * 1024;
 
-  // First step straight from its task record.
+  // First step straight from its task record.  A work-group past the first
+  // chunks finds its step in the list instead.
   Step cur;
+  cur.q = blockIdx.x;
   cur.j = blockIdx.x / ntp;
-  if (cur.j >= a.max_active) return;
-  const int32_t* tk0 = a.tasks + static_cast<size_t>(cur.j) * kTaskInts;
-  cur.e = tk0[0];
-  if (cur.e < 0) return;
-  cur.off = tk0[1];
-  cur.M = tk0[2];
+  const int32_t* tk0 = a.tasks + static_cast<size_t>(min(cur.j, a.max_active - 1)) * kTaskInts;
+  cur.e = __builtin_amdgcn_readfirstlane(tk0[0]);
+  cur.off = __builtin_amdgcn_readfirstlane(tk0[1]);
+  cur.M = __builtin_amdgcn_readfirstlane(tk0[2]);
   cur.tp = blockIdx.x - cur.j * ntp;
   cur.c = 0;
-  cur.valid = 1;
+  cur.valid = cur.j < a.max_active && cur.e >= 0;
+  const bool direct = cur.valid;
 
-  // Task headers into LDS (issued first: their wait leaves the rest in flight).
-  int4 hv = make_int4(-1, 0, 0, 0);
-  if (static_cast<int>(threadIdx.x) < a.max_active)
-    hv = reinterpret_cast<const int4*>(a.tasks)[static_cast<size_t>(threadIdx.x) * (kTaskInts / 4)];
-  static_assert(kMaxExperts <= 256, "expert id packs into 8 bits");
-  const int nact = *a.n_active;
-  // Small batches stage the slot -> token map (S <= kTok) so the next step's
-  // token ids are LDS reads rather than loads queued behind the weights.
-  int tv = 0;
-  if constexpr (kGated && kTok > 1)
-    if (static_cast<int>(threadIdx.x) < a.slots) tv = a.perm_token[threadIdx.x];
+  // Task headers (wave 0; issued first: their wait leaves the rest in flight).
+  static_assert(kMaxExperts % kWave == 0 && kMaxExperts <= 256, "whole waves of records, expert id packs into 8 bits");
+  constexpr int kRec = kMaxExperts / kWave;
+  int4 hv[kRec];
+  if (p == 0) {
+#pragma unroll
+    for (int i = 0; i < kRec; ++i) {
+      const int r = lane + i * kWave;
+      hv[i] = make_int4(-1, 0, 0, 0);
+      if (r < a.max_active) hv[i] = reinterpret_cast<const int4*>(a.tasks)[static_cast<size_t>(r) * (kTaskInts / 4)];
+    }
+  }
+  const int nact = __builtin_amdgcn_readfirstlane(*a.n_active);
+  const int nfirst = nact * ntp;
+  auto publish = [&]() {
+    if (p == 0) {
+      int base = 0;
+#pragma unroll
+      for (int i = 0; i < kRec; ++i) {
+        const int r = lane + i * kWave;
+        sm.hdr[r] = make_int2(hv[i].x < 0 ? -1 : (hv[i].x | (hv[i].z << 8)), hv[i].y);
+        int n = hv[i].x < 0 ? 0 : (hv[i].z - 1) / TC;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+          const int u = __shfl_up(n, d, kWave);
+          n += lane >= d ? u : 0;
+        }
+        sm.more[r] = base + n;
+        base += __shfl(n, kWave - 1, kWave);
+      }
+    }
+    __syncthreads();
+  };
+  auto step_of = [&](int q) -> Step {
+    Step n;
+    n.q = q;
+    n.c = 0;
+    if (q < nfirst) {
+      n.j = q / ntp;
+      n.tp = q - n.j * ntp;
+    } else {
+      const int x = (q - nfirst) / ntp;  // the x-th further chunk
+      n.tp = q - nfirst - x * ntp;
+      n.j = 0;
+#pragma unroll
+      for (int i = 0; i < kRec; ++i) n.j += __popcll(__ballot(sm.more[lane + i * kWave] <= x));
+      if (n.j < nact) n.c = 1 + x - (n.j ? __builtin_amdgcn_readfirstlane(sm.more[n.j - 1]) : 0);
+    }
+    n.valid = n.j < nact;
+    const int2 h = sm.hdr[n.valid ? n.j : 0];
+    const int hx = __builtin_amdgcn_readfirstlane(h.x);
+    n.valid = n.valid && hx >= 0;
+    n.e = hx & 0xff;
+    n.M = hx >> 8;
+    n.off = __builtin_amdgcn_readfirstlane(h.y);
+    return n;
+  };
+  if (!direct) {
+    publish();
+    cur = step_of(blockIdx.x);
+    if (!cur.valid) return;
+  }
 
   // Per-step addresses (dwords; a block is 256 of them).  An invalid step
   // points every load at fixed valid data (expert 0, tile 0, input row 0)
@@ -263,8 +319,26 @@ void expert_stream_kernel(StreamParams a) {
   // Prologue: the first step's scales, activations and first kD blocks.
   uint32_t sc[R][kMaxBpp / 4];
   load_sc(cur, sc);
+  // Token ids of a step's activation slots (gate_up).
+  auto tokens_of = [&](const Step& s, int (&tok)[kN]) {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) tok[i] = 0;
+    if constexpr (kGated) {
+      const int mc = s.valid ? min(TC, s.M - s.c * TC) : 1;
+#pragma unroll
+      for (int i = 0; i < kN; ++i) {
+        int m, c;
+        slot_of<TC>(i, lane, mc, nchunk, m, c);
+        const int mg = s.c * TC + m;
+        const int32_t* tp = !s.valid ? a.tasks
+                            : mg < kTaskTokens ? a.tasks + static_cast<size_t>(s.j) * kTaskInts + 4 + mg
+                                               : a.perm_token + s.off + mg;
+        tok[i] = *tp;
+      }
+    }
+  };
   int tok[kN];
-  if constexpr (kGated) {
+  if (kGated && direct) {
     // the first chunk's tokens are all inline in the record (TC <= kTaskTokens)
     static_assert(TC <= kTaskTokens, "first chunk must fit the inline tokens");
     int t0[TC];
@@ -281,8 +355,7 @@ void expert_stream_kernel(StreamParams a) {
       tok[i] = t;
     }
   } else {
-#pragma unroll
-    for (int i = 0; i < kN; ++i) tok[i] = 0;
+    tokens_of(cur, tok);
   }
   XSlots<TC, PK> xl;
   issue_x(cur, tok, xl);
@@ -297,67 +370,15 @@ void expert_stream_kernel(StreamParams a) {
         if (BPP || i < bpp) ring[r][i] = load_slot_nt(src + static_cast<size_t>(i) * stride);
     }
   }
-  if (static_cast<int>(threadIdx.x) < kMaxExperts)
-    sm.hdr[threadIdx.x] = make_int2(hv.x < 0 ? -1 : (hv.x | (hv.z << 8)), hv.y);
-  // A block of 64 x parts threads holds fewer threads than records when K
-  // splits into one to three parts and more experts are active: the rest of
-  // the records, here (their wait also covers the weight loads above).
-  for (int i = static_cast<int>(threadIdx.x + blockDim.x); i < min(a.max_active, kMaxExperts);
-       i += static_cast<int>(blockDim.x)) {
-    const int4 h = reinterpret_cast<const int4*>(a.tasks)[static_cast<size_t>(i) * (kTaskInts / 4)];
-    sm.hdr[i] = make_int2(h.x < 0 ? -1 : (h.x | (h.z << 8)), h.y);
-  }
-  if constexpr (kGated && kTok > 1)
-    if (static_cast<int>(threadIdx.x) < a.slots) sm.tok[threadIdx.x] = tv;
-  __syncthreads();
+  if (direct) publish();
 
-  store_x<TC, PK>(xl, sm.x[p], min(TC, cur.M), nchunk, lane);
-
-  auto next_of = [&](const Step& s) -> Step {
-    Step n;
-    if ((s.c + 1) * TC < s.M) {
-      n = s;
-      n.c = s.c + 1;
-      return n;
-    }
-    const int q = (s.j * ntp + s.tp) + G;
-    n.j = q / ntp;
-    n.tp = q - n.j * ntp;
-    n.c = 0;
-    n.valid = n.j < nact;
-    const int2 h = sm.hdr[n.valid ? n.j : 0];
-    n.valid = n.valid && h.x >= 0;
-    n.e = h.x & 0xff;
-    n.M = h.x >> 8;
-    n.off = h.y;
-    return n;
-  };
+  store_x<TC, PK>(xl, sm.x[p], min(TC, cur.M - cur.c * TC), nchunk, lane);
 
   for (;;) {
-    const Step nxt = next_of(cur);
-    // token ids of the next step's activation slots (gate_up): small loads
-    // that land long before the next step's activations are issued
+    const Step nxt = step_of(cur.q + G);
+    // small loads that land long before the next step's activations are issued
     int ntok[kN];
-    if constexpr (kGated) {
-      const int mc = nxt.valid ? min(TC, nxt.M - nxt.c * TC) : 1;
-#pragma unroll
-      for (int i = 0; i < kN; ++i) {
-        int m, c;
-        slot_of<TC>(i, lane, mc, nchunk, m, c);
-        const int mg = nxt.c * TC + m;
-        if constexpr (kTok > 1) {
-          ntok[i] = nxt.valid ? sm.tok[nxt.off + mg] : 0;
-        } else {
-          const int32_t* tp = !nxt.valid ? a.tasks
-                              : mg < kTaskTokens ? a.tasks + static_cast<size_t>(nxt.j) * kTaskInts + 4 + mg
-                                                 : a.perm_token + nxt.off + mg;
-          ntok[i] = *tp;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kN; ++i) ntok[i] = 0;
-    }
+    tokens_of(nxt, ntok);
     const int mc = __builtin_amdgcn_readfirstlane(min(TC, cur.M - cur.c * TC));
     const float(*sx)[PK] = sm.x[p];
     int cstride[R], nstride[R];
@@ -602,43 +623,42 @@ __global__ void pack_mscale_kernel(const uint8_t* __restrict__ src, int N, int n
 
 }  // namespace
 
-// Launch shapes.  Decode batches of up to 64 routed slots (8 tokens at
-// top-4) put one row on each lane (the most work-groups for a latency-bound
-// step) and stage the slot -> token map in LDS; larger batches put two
-// rows on each lane (half the LDS activation traffic per FMA) and stage 4
-// tokens per step.  The grid never exceeds the items a launch can have
-// (max_active x tile groups) nor what stays resident on the device.
-template <int BPP, int R, int TC, int D, bool kGated, int kTok>
-static void launch_stream_t(const ExpertArgs& a, const TiledGeom& g, bool gated, hipStream_t s) {
+// Launch shapes.  Two rows on each lane halve the LDS activation traffic per
+// fmaf and a chunk of four tokens the weight decode; a batch of up to 8 routed
+// slots (2 tokens at top-4) has at most a few steps per work-group and waits
+// for latency, so it takes one row per lane (twice the steps) and three
+// work-groups per CU instead of two.  A 20B layer of 1 / 2 / 4 / 8
+// tokens: one row 35 / 47 / 68 / 104 us, two rows 41 / 52 / 64 / 87 us.  The grid never exceeds the steps a
+// launch can have (first chunks: max_active x tile groups; further ones: at
+// most one per TC slots) nor what stays resident on the device.
+template <int BPP, int R, int TC, int D, bool kGated>
+static void launch_stream_t(const ExpertArgs& a, const TiledGeom& g, hipStream_t s) {
   StreamParams p{};
-  p.x = gated ? a.x : a.act;
-  p.wn = gated ? a.w1n : a.w2n;
-  p.ws = gated ? a.w1s : a.w2s;
-  p.bias = gated ? a.b1 : a.b2;
+  p.x = kGated ? a.x : a.act;
+  p.wn = kGated ? a.w1n : a.w2n;
+  p.ws = kGated ? a.w1s : a.w2s;
+  p.bias = kGated ? a.b1 : a.b2;
   p.tasks = a.plan.tasks;
   p.n_active = a.plan.n_active;
   p.perm_token = a.plan.perm_token;
-  p.slots = a.T * a.k;
-  p.out = gated ? a.act : a.y;
-  p.gate_up = gated ? a.gate_up : nullptr;
+  p.out = kGated ? a.act : a.y;
+  p.gate_up = kGated ? a.gate_up : nullptr;
   p.max_active = a.max_active;
   p.alpha = a.alpha;
   p.limit = a.limit;
   p.g = g;
   const int ntp = (g.N / kTileRows + R - 1) / R;
-  const int items = a.max_active * ntp;
-  const int resident = 256 * 2;
+  const int items = (a.max_active + a.T * a.k / TC) * ntp;
+  const int resident = 256 * (R == 1 ? 3 : 2);
   const int grid = items < resident ? items : resident;
-  gx_launch(expert_stream_kernel<BPP, R, TC, D, kGated, kTok>, dim3(grid), dim3(kTileRows * g.parts), 0, s, a.timer,
-            p);
+  gx_launch(expert_stream_kernel<BPP, R, TC, D, kGated>, dim3(grid), dim3(kTileRows * g.parts), 0, s, a.timer, p);
 }
 
 template <int BPP, bool kGated>
 static void launch_stream_b(const ExpertArgs& a, const TiledGeom& g, hipStream_t s) {
-  constexpr int kLoop = BPP ? BPP : kMaxBpp;
-  if (a.T * a.k <= 16) launch_stream_t<BPP, 1, 2, kLoop, kGated, 64>(a, g, kGated, s);
-  else if (a.T * a.k <= 64) launch_stream_t<BPP, 1, 2, (kLoop % 5 == 0 ? 5 : kLoop), kGated, 64>(a, g, kGated, s);
-  else launch_stream_t<BPP, 2, 4, (kLoop % 3 == 0 ? 3 : kLoop), kGated, 1>(a, g, kGated, s);
+  constexpr int D = BPP == 15 ? 3 : BPP == 1 ? 1 : 4;
+  if (a.T * a.k <= 8) launch_stream_t<BPP, 1, 4, D, kGated>(a, g, s);
+  else launch_stream_t<BPP, 2, 4, D, kGated>(a, g, s);
 }
 
 // Blocks per K-part: 15 for K = 2880 (GPT-OSS), 1 for small K; any other

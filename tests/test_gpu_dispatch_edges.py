@@ -1,7 +1,7 @@
 """Sizes at the edges of the dispatch rules, against the oracle or a plain
 restatement: the dense GEMV's rows per work-group, unaligned inputs and scale
 codes 0 and 255; the layer's routing plan around the sizes where its launches
-change."""
+change; the exact decode's steps under skewed routing."""
 import numpy as np
 import pytest
 import torch
@@ -84,4 +84,34 @@ def test_layer_plan(E, k, T):
     assert np.array_equal(read(tr.gather_map, S), gmap)
     assert np.array_equal(read(tr.perm_token, S), order // k)
     assert read(tr.n_active, 1)[0] == act.size and np.array_equal(read(tr.active_experts, E)[:act.size], act)
+    layer.destroy()
+
+
+# exact decode under skewed routing, token for token the bits of a batch of
+# one: K-parts of an odd and an even number of blocks, one to six of them; one row per lane (up to 8
+# slots) or two; more and fewer first chunks than work-groups, experts from
+# one token to all of them, more records than one wave holds
+@pytest.mark.parametrize("E,k,H,I", [(1, 1, 128, 64), (30, 4, 448, 192), (200, 4, 128, 64), (8, 2, 2880, 960)])
+@pytest.mark.parametrize("T", [1, 2, 3, 17, 64, 150])
+def test_exact_steps(E, k, H, I, T):
+    w = moe_data.make_layer(3, E, H, I, bias="random")
+    x, res = moe_data.make_tokens(T, T, H)
+    cfg = g.default_config(E, T, decode_exact=True, prefill_min_tokens=0)
+    cfg.hidden_size, cfg.intermediate_size, cfg.top_k = H, I, k
+    t = {n: _dev(v) for n, v in w.items()}
+    layer = g.MoELayer().init(cfg, 0, t["router_w"], t["router_b"], t["w1_bias"], t["w2_bias"],
+                              mlp1=([t["w1_packed"][e] for e in range(E)], [t["w1_scales"][e] for e in range(E)]),
+                              mlp2=([t["w2_packed"][e] for e in range(E)], [t["w2_scales"][e] for e in range(E)]))
+    rng = np.random.default_rng([E, T])
+    # expert 0 of every token, the others by a steep law
+    p = 1.0 / np.arange(1, E) ** 1.3
+    rest = [rng.choice(np.arange(1, E), k - 1, replace=False, p=p / p.sum()) if k > 1 else [] for _ in range(T)]
+    idx = _dev(np.array([[0, *r] for r in rest], dtype=np.int32))
+    wts = _dev(rng.dirichlet(np.ones(k), T).astype(np.float32))
+    dx, dr = _dev(x), _dev(res)
+    got = _bits(layer.forward_routed(dx, idx, wts, residual=dr))
+    for i in range(T):
+        one = layer.forward_routed(dx[i:i + 1].contiguous(), idx[i:i + 1].contiguous(), wts[i:i + 1].contiguous(),
+                                   residual=dr[i:i + 1].contiguous())
+        assert np.array_equal(_bits(one)[0], got[i]), i
     layer.destroy()
