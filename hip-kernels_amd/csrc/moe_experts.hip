@@ -681,12 +681,16 @@ hipError_t launch_w2(const ExpertArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t launch_combine8(uint16_t* out, const uint16_t* y, const int32_t* gather_map, const float* w,
+                           const uint16_t* residual, int T, int H, int k, KernelTimer timer, hipStream_t s) {
+  const int n = T * (H / 8);
+  gx_launch(combine8_kernel, dim3((n + 255) / 256), dim3(256), 0, s, timer, y, gather_map, w, residual, out, T, H, k);
+  return hipGetLastError();
+}
+
 hipError_t launch_combine_slots(const ExpertArgs& a, hipStream_t s) {
   if (a.T <= 0) return hipSuccess;
-  const int n = a.T * (a.H / 8);
-  gx_launch(combine8_kernel, dim3((n + 255) / 256), dim3(256), 0, s, a.timer, static_cast<const uint16_t*>(a.y),
-            static_cast<const int32_t*>(a.plan.gather_map), a.w, a.residual, a.out, a.T, a.H, a.k);
-  return hipGetLastError();
+  return launch_combine8(a.out, a.y, a.plan.gather_map, a.w, a.residual, a.T, a.H, a.k, a.timer, s);
 }
 
 hipError_t launch_experts(const ExpertArgs& a, hipStream_t s) {

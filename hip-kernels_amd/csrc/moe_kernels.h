@@ -174,6 +174,10 @@ hipError_t launch_experts(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_w1(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_w2(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_combine_slots(const ExpertArgs& a, hipStream_t s);
+// H a multiple of 8, rows of out, y and residual (may be null) on 16 bytes,
+// T * H / 8 below 2^30.
+hipError_t launch_combine8(uint16_t* out, const uint16_t* y, const int32_t* gather_map, const float* w,
+                           const uint16_t* residual, int T, int H, int k, KernelTimer timer, hipStream_t s);
 // The decode expert products on the matrix cores (moe_decode.hip): same
 // outputs as launch_w1 / launch_w2 up to fp32 summation order.
 hipError_t launch_w1_mc(const ExpertArgs& a, hipStream_t s);

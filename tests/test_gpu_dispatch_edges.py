@@ -1,7 +1,8 @@
 """Sizes at the edges of the dispatch rules, against the oracle or a plain
 restatement: the dense GEMV's rows per work-group, unaligned inputs and scale
 codes 0 and 255; the layer's routing plan around the sizes where its launches
-change; the exact decode's steps under skewed routing."""
+change; the exact decode's steps under skewed routing; the stage
+combine's 16-byte form and its fallback."""
 import numpy as np
 import pytest
 import torch
@@ -115,3 +116,28 @@ def test_exact_steps(E, k, H, I, T):
                                    residual=dr[i:i + 1].contiguous())
         assert np.array_equal(_bits(one)[0], got[i]), i
     layer.destroy()
+
+
+def _shifted(a, shift):
+    """The rows of a on the device, `shift` elements past a 16-byte boundary."""
+    t = _dev(a)
+    buf = torch.zeros(t.numel() + 16, dtype=t.dtype, device="cuda")
+    v = buf[shift:shift + t.numel()].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+# 16-byte pieces or one output per thread; dropped slots; every top-k
+@pytest.mark.parametrize("T,H,k", [(1, 8, 1), (5, 20, 3), (33, 64, 8), (257, 2888, 4)])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("residual", [True, False])
+def test_combine_forms(T, H, k, shift, residual):
+    rng = np.random.default_rng([T, H, k])
+    S = T * k
+    y, res = moe_data.bf16(rng.normal(0, 1, (S, H))), moe_data.bf16(rng.normal(0, 1, (T, H)))
+    gm = rng.permutation(S).astype(np.int32)
+    if S > 4:
+        gm[rng.choice(S, S // 5, replace=False)] = -1
+    w = rng.dirichlet(np.ones(k), T).astype(np.float32)
+    got = _bits(g.combine(_shifted(y, shift), _dev(gm), _dev(w), _dev(res) if residual else None, T, H, k))
+    assert np.array_equal(got, orc.combine(y, gm, w, res if residual else None, T, k, H))
