@@ -10,9 +10,10 @@
 //   expert_stream_kernel<!gated>  down: + bias, bf16 expert outputs
 //   combine8_kernel               out = bf16(sum_k w_k * y_k + residual)
 //
-// The stream kernel is persistent: at most two work-groups per CU walk the
-// (active expert, tile group) items of the routing plan's task records, so
-// the weights stream without a gap between items (see expert_stream_kernel).
+// The stream kernel is persistent: at most two work-groups per CU (three up to
+// 8 slots) walk the (active expert, tile group, token chunk) steps of the
+// routing plan's task records, so the weights stream without a gap between
+// steps (see expert_stream_kernel).
 //
 // Memory layout (tiled MXFP4, built once by pack_nib/pack_scale; TiledGeom
 // in moe_kernels.h): for each expert, each 64-row tile holds nb = K/32 blocks
@@ -150,10 +151,10 @@ struct Step {
 // likewise.  (A chunk reads its weights again either way, so a work-group that
 // kept all chunks of its tiles only made the busiest expert the longest wait:
 // 24 tokens, 32 experts, both launches: Zipf routing 380 us so and 170 as
-// single steps, uniform routing 192 and 166.)  Lane l of wave p owns row l of each tile and runs, per
-// token, one ascending fmaf chain over K-part p (the canonical dot); the part
-// sums are added in part order across the work-group, which then adds the
-// bias and emits (gate_up: bf16 gate/up values, clamped SwiGLU on lane pairs,
+// single steps, uniform routing 192 and 166.)  Lane l of wave p owns row l of
+// each tile and runs, per token, one ascending fmaf chain over K-part p (the
+// canonical dot); the part sums are added in part order across the work-group,
+// which then adds the bias and emits (gate_up: bf16 gate/up values, clamped SwiGLU on lane pairs,
 // bf16 activations; down: bf16 expert outputs).
 //
 // Streaming: the weights of a step move through a ring of D blocks per row
@@ -627,10 +628,11 @@ __global__ void pack_mscale_kernel(const uint8_t* __restrict__ src, int N, int n
 // fmaf and a chunk of four tokens the weight decode; a batch of up to 8 routed
 // slots (2 tokens at top-4) has at most a few steps per work-group and waits
 // for latency, so it takes one row per lane (twice the steps) and three
-// work-groups per CU instead of two.  A 20B layer of 1 / 2 / 4 / 8
-// tokens: one row 35 / 47 / 68 / 104 us, two rows 41 / 52 / 64 / 87 us.  The grid never exceeds the steps a
-// launch can have (first chunks: max_active x tile groups; further ones: at
-// most one per TC slots) nor what stays resident on the device.
+// work-groups per CU instead of two.  A 20B layer of 1 / 2 / 4 / 8 tokens:
+// one row 35 / 47 / 68 / 104 us, two rows 41 / 52 / 64 / 87 us.  The grid
+// never exceeds the steps a launch can have (first chunks: max_active x tile
+// groups; further ones: at most one per TC slots) nor what stays resident on
+// the device.
 template <int BPP, int R, int TC, int D, bool kGated>
 static void launch_stream_t(const ExpertArgs& a, const TiledGeom& g, hipStream_t s) {
   StreamParams p{};
