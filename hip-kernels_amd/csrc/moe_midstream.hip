@@ -174,6 +174,10 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
     return srow < s.mc ? static_cast<uint32_t>(s.p0 + srow) * 4u : a.idx_bytes;
   };
   const bool gather = a.row_index != nullptr;
+  // Scalar offset of K block b.  The range check compares the lane's offset
+  // with the extent less the scalar offset, so the latter stays within the
+  // extent: 0 for a block past K, which with one row of x would lie past it.
+  auto xblk = [&](int b) -> int { return b < nb ? 64 * b : 0; };
 
   gx_u32x4 ra[PB];   // the weight ring: slot i = block i of the phase being (or next) consumed
   gx_u32x4 xt[PB];   // a phase's tokens on their way to LDS
@@ -201,7 +205,7 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
     // the second phase's tokens stay in flight: phase p writes phase p + 1's
 #pragma unroll
     for (int r = 0; r < PB; ++r)
-      xt[r] = __builtin_amdgcn_raw_buffer_load_b128(rX, PB + r < nb ? vx : a.x_bytes, 64 * (PB + r), 0);
+      xt[r] = __builtin_amdgcn_raw_buffer_load_b128(rX, PB + r < nb ? vx : a.x_bytes, xblk(PB + r), 0);
     scs[w][0][min(lane, 4 * PB)] = sv;
     spec = lv && lane < 4 * min(PB, nb) && any_special(sv);
   }
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
             for (int r = kIssue * (i - PB + 1 + kLead); r < kIssue * (i - PB + 2 + kLead) && r < PB; ++r) {
               *reinterpret_cast<gx_u32x4*>(xwr + 1024 * NC * r) = xt[r];
               xt[r] = __builtin_amdgcn_raw_buffer_load_b128(rX, xb0 + r < nb ? (xnext ? vxn : vx) : a.x_bytes,
-                                                            64 * (xb0 + r), 0);
+                                                            xblk(xb0 + r), 0);
             }
           }
           if (i == PB - 3) {

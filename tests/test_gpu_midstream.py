@@ -68,6 +68,52 @@ def test_mid_stream_rows(N, K, counts, special):
         assert (np.abs(y[r] - want) <= bound).all()
 
 
+def _nan_behind(a):
+    """The rows of a on the device, followed by NaN."""
+    t = _dev(a)
+    buf = torch.full((t.numel() + 8192,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    v = buf[:t.numel()].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+# One row of x: a phase's loads of K blocks past the last must not reach
+# behind the row, where NaN would survive the zero weights.
+@pytest.mark.parametrize("K", [320, 352, 416, 576, 1024, 1056])
+def test_mid_stream_one_row_of_x(K):
+    E, N = 2, 128
+    rng = np.random.default_rng(K)
+    packed = rng.integers(0, 256, (E, N, K // 2), dtype=np.uint8)
+    scales = rng.integers(119, 124, (E, N, K // 32), dtype=np.uint8)
+    x = moe_data.bf16(rng.normal(0.0, 1.0, (1, K)))
+    tn, ts = _tiled((packed, scales), E, N, K)
+    offs = torch.tensor([0, 0, 1], dtype=torch.int32, device="cuda")
+    y = g.grouped_mxfp4_gemm(_nan_behind(x), offs, tn, ts, N, K, 1).float().cpu().numpy()
+    xf = orc.bf16_to_f32(x).astype(np.float64)
+    w = _dequant(packed[1], scales[1])
+    bound = 2.0 ** -8 * np.abs(xf @ w.T) + (K + 2) * 2.0 ** -24 * (np.abs(xf) @ np.abs(w).T + 1.0)
+    assert (np.abs(y - xf @ w.T) <= bound).all()
+
+
+# The same through the layer, which gathers its one token for every expert.
+def test_mid_stream_one_token_layer():
+    E, k, H, I = 8, 4, 320, 448
+    w = moe_data.make_layer(3, E, H, I, bias="random")
+    x, res = moe_data.make_tokens(1, 1, H)
+    cfg = g.default_config(E, 1, prefill_min_tokens=1)
+    cfg.hidden_size, cfg.intermediate_size, cfg.top_k = H, I, k
+    t = {n: _dev(v) for n, v in w.items()}
+    layer = g.MoELayer().init(cfg, 0, t["router_w"], t["router_b"], t["w1_bias"], t["w2_bias"],
+                              mlp1=([t["w1_packed"][e] for e in range(E)], [t["w1_scales"][e] for e in range(E)]),
+                              mlp2=([t["w2_packed"][e] for e in range(E)], [t["w2_scales"][e] for e in range(E)]))
+    idx = torch.tensor([[5, 0, 7, 2]], dtype=torch.int32, device="cuda")
+    wts = torch.tensor([[0.4, 0.3, 0.2, 0.1]], device="cuda")
+    a = layer.forward_routed(_dev(x), idx, wts, residual=_dev(res))
+    b = layer.forward_routed(_nan_behind(x), idx, wts, residual=_dev(res))
+    assert torch.isfinite(a.float()).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
+    layer.destroy()
+
+
 def _dequant(packed, scales):
     lut = np.array([0, 0.5, 1, 1.5, 2, 3, 4, 6, -0.0, -0.5, -1, -1.5, -2, -3, -4, -6])
     v = np.stack([lut[packed & 15], lut[packed >> 4]], axis=-1).reshape(packed.shape[0], -1)
