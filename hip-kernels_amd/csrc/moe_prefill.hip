@@ -1065,7 +1065,6 @@ bool grouped_supported(int N, int K, int E) {
 hipError_t launch_grouped_mxfp4(const GroupedArgs& a, hipStream_t s) {
   if (a.rows <= 0) return hipSuccess;
   if (!grouped_supported(a.N, a.K, a.E)) return hipErrorInvalidValue;
-  if (mid_stream_pays(a) && mid_stream_supported(a)) return launch_mid_stream(a, s);
   GroupedParams p{};
   p.x = a.x;
   p.row_index = a.row_index;
@@ -1099,6 +1098,7 @@ hipError_t launch_grouped_mxfp4(const GroupedArgs& a, hipStream_t s) {
   if (per_xcd > (1L << 27) || fb >= (1L << 16) * p.nwt || static_cast<size_t>(a.N) * (a.K / 32) > (1u << 30) ||
       p.g.nib_bytes >= (static_cast<size_t>(1) << 31))
     return hipErrorInvalidValue;  // tile counts (16-bit scan fields) and buffer offsets (32-bit)
+  if (mid_stream_pays(a) && mid_stream_supported(a)) return launch_mid_stream(a, s);
   int grid = static_cast<int>(8 * per_xcd);
   if (mx) {
     const int slots = 8 * ((a.num_cus + 7) / 8);  // one work-group per CU, a multiple of 8

@@ -114,6 +114,21 @@ def test_mid_stream_one_token_layer():
     layer.destroy()
 
 
+# What the grouped product refuses (an expert's nibbles of 2 GiB or more) it
+# refuses at every row count.  The buffers are real: nothing would be read out
+# of range if a call were taken.
+@pytest.mark.parametrize("rows", [1, 40, 1801])
+def test_matrix_too_large_is_refused(rows):
+    N, K = 1398144, 3072
+    nb, sb = g.tiled_size(N, K)
+    assert nb >= 2 ** 31
+    nib, sc = (torch.zeros(n, dtype=torch.uint8, device="cuda") for n in (nb, sb))
+    x = torch.zeros((rows, K), dtype=torch.bfloat16, device="cuda")
+    offs = torch.zeros(2, dtype=torch.int32, device="cuda")
+    with pytest.raises(g.GptossError, match="grouped gemm launch"):
+        g.grouped_mxfp4_gemm(x, offs, nib, sc, N, K, rows)
+
+
 def _dequant(packed, scales):
     lut = np.array([0, 0.5, 1, 1.5, 2, 3, 4, 6, -0.0, -0.5, -1, -1.5, -2, -3, -4, -6])
     v = np.stack([lut[packed & 15], lut[packed >> 4]], axis=-1).reshape(packed.shape[0], -1)
