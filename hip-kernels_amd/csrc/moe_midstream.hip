@@ -8,8 +8,8 @@
 // is a weight stream like the decode kernel's, with the tokens in LDS:
 //
 // * An item is (chunk of up to 64 rows of one expert) x (four 64-row weight
-//   tiles); a work-group of four waves, a tile each, takes items v, v + G, ...
-//   (v: the XCD-grouped block index, so an XCD's work-groups share an expert's
+//   tiles); a work-group of four waves, a tile each, takes one item of every
+//   round of G (grouped by XCD, so an XCD's work-groups share an expert's
 //   token rows in L2).  Two work-groups run per CU (registers and LDS).
 // * Each wave streams its tile's 1 KiB blocks with 16-byte nontemporal loads
 //   into a ring of PB register slots: consuming block i of a phase (PB
@@ -61,7 +61,7 @@ struct MidParams {
   uint16_t* out;             // gated: [rows][N/2] activations; else [rows][N]
   uint16_t* gate_up;         // gated and optional: [rows][N] bf16 gate/up values
   uint32_t x_bytes, idx_bytes, wn_bytes, ws_bytes, bias_bytes, out_bytes;  // buffer extents (each < 2^32 - 2^16)
-  int E;
+  int E, num_cus;
   float alpha, limit;
   TiledGeom g;
 };
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
   __shared__ gx_u32x4 scs[kMidWaves][2][PB * 4 + 1];
   __shared__ uint2 bs[kMidWaves][kTileRows / 4 + 1];
   __shared__ int2 tab[kMidChunks];                // chunks: {expert | rows << 8, first permuted row}
-  __shared__ int tab_n;
+  __shared__ int tab_n, tail_item;
 
   const TiledGeom& g = a.g;
   const int lane = threadIdx.x & 63;
@@ -126,9 +126,28 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
   }
   __syncthreads();
   const int n_items = min(__builtin_amdgcn_readfirstlane(tab_n), kMidChunks) * ngrp;
-  const int G = gridDim.x;  // a multiple of 8: block b runs on XCD b % 8
-  int q = (static_cast<int>(blockIdx.x) & 7) * (G >> 3) + (static_cast<int>(blockIdx.x) >> 3);
-  if (q >= n_items) return;
+  // Items go in rounds of G, XCD b % 8 taking consecutive ones.  A last round
+  // of at most one item per CU is dealt evenly to the XCDs: packed into the
+  // first of them, 92 items (200 rows on four experts) ran on two XCDs in
+  // 48 us, spread over eight in 33, and the 128 left of 1664 (200 rows on 128
+  // experts) cost 157 us against 138.  A fuller one stays packed: it puts two
+  // work-groups on most CUs either way (2944 items: 193 us, spread 194).
+  const int G = gridDim.x;  // a multiple of 8
+  const int full = n_items / G * G;  // items of the full rounds
+  int q;                             // this work-group's item, -1: none
+  {
+    const int xcd = static_cast<int>(blockIdx.x) & 7, slot = static_cast<int>(blockIdx.x) >> 3;
+    const int left = n_items - full;
+    const int share = left > a.num_cus ? G >> 3 : (left + 7) >> 3;
+    const int o = xcd * share + slot;
+    const int tail = slot < share && o < left ? full + o : -1;
+    if (threadIdx.x == 0) tail_item = tail;
+    q = full > 0 ? xcd * (G >> 3) + slot : tail;
+  }
+  if (q < 0) return;
+  auto next_item = [&]() -> int {
+    return q + G < full ? q + G : q < full ? __builtin_amdgcn_readfirstlane(tail_item) : -1;
+  };
 
   const __amdgpu_buffer_rsrc_t rX = rsrc_of(a.x, a.x_bytes);
   const __amdgpu_buffer_rsrc_t rI = rsrc_of(a.row_index, a.idx_bytes);
@@ -139,7 +158,7 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
 
   auto item_of = [&](int qq) -> MidItem {
     MidItem s;
-    s.valid = qq < n_items;
+    s.valid = qq >= 0;
     const int j = s.valid ? qq / ngrp : 0;
     s.tile = (qq - j * ngrp) * kMidWaves + w;
     const int hx = __builtin_amdgcn_readfirstlane(tab[j].x);
@@ -227,7 +246,8 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
   }
 
   for (;;) {
-    const MidItem nxt = item_of(q + G);
+    q = next_item();
+    const MidItem nxt = item_of(q);
     uint32_t vxn = 0;    // the next item's token row
     bool nspec = false;  // special codes seen in the next item's first phase
     {
@@ -404,7 +424,6 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
     cur = nxt;
     vx = vxn;
     spec = nspec;
-    q += G;
   }
 }
 
@@ -460,6 +479,7 @@ hipError_t launch_mid_stream(const GroupedArgs& a, hipStream_t s) {
   p.bias_bytes = a.bias ? static_cast<uint32_t>(static_cast<size_t>(a.E) * a.N * 2) : 0u;
   p.out_bytes = static_cast<uint32_t>(static_cast<size_t>(a.rows) * (a.gated ? a.N / 2 : a.N) * 2);
   p.E = a.E;
+  p.num_cus = a.num_cus;
   p.alpha = a.alpha;
   p.limit = a.limit;
   const int ngrp = (a.N / kTileRows + kMidWaves - 1) / kMidWaves;

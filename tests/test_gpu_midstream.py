@@ -114,6 +114,96 @@ def test_mid_stream_one_token_layer():
     layer.destroy()
 
 
+def _random_tiled(E, N, K, special, seed):
+    """Uniform codes and scales, made on the device; special: codes 0 and 255
+    in the scales of every fifth expert."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    nb, sb = g.tiled_size(N, K)
+    out = torch.empty(E * nb, dtype=torch.uint8, device="cuda"), torch.empty(E * sb, dtype=torch.uint8, device="cuda")
+    for e in range(E):
+        q = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device="cuda", generator=gen)
+        s = torch.randint(119, 124, (N, K // 32), dtype=torch.uint8, device="cuda", generator=gen)
+        if special and e % 5 == 0:
+            s[e % N, -1], s[(7 * e + 70) % N, e % (K // 32)] = 0, 255
+        g.pack_tiled(q, s, N, K, out[0][e * nb:(e + 1) * nb], out[1][e * sb:(e + 1) * sb])
+    return out
+
+
+# Several items per work-group (about 130 chunks x 8 groups of tiles on 512
+# work-groups: full rounds and a partial one), and fewer items than
+# work-groups; phases of 8 (K / 32 = 16, 22) and 9 blocks (18, 26), two and
+# three of them; chunks of 1 to 64 rows next to each other
+@pytest.mark.parametrize("K", [512, 576, 704, 832])
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("routing", ["ragged", "few"])
+def test_mid_stream_many_items(K, special, routing):
+    E, N = 96, 2048
+    rng = np.random.default_rng([K, special])
+    counts = np.zeros(E, dtype=np.int64)
+    if routing == "ragged":
+        counts[:] = rng.choice([0, 1, 5, 8, 16, 17, 31, 33], E, p=[.15, .15, .15, .15, .12, .12, .08, .08])
+        counts[rng.choice(E, 6, replace=False)] = [47, 49, 63, 64, 65, 100]
+    else:
+        counts[rng.choice(E, 4, replace=False)] = [50, 50, 16, 129]
+    S = int(counts.sum())
+    assert S <= 1800
+    tn, ts = _random_tiled(E + 1, N, K, special, K)
+    gen = torch.Generator(device="cuda").manual_seed(K + 1)
+    x = torch.randn((S + 1801, K), device="cuda", generator=gen).to(torch.bfloat16)
+    bias = (0.5 * torch.randn((E + 1, N), device="cuda", generator=gen)).to(torch.bfloat16)
+    offs = np.concatenate([[0], np.cumsum(counts)])
+    small, large = _dev(np.append(offs, S).astype(np.int32)), _dev(np.append(offs, S + 1801).astype(np.int32))
+    for swiglu, b in ((False, bias), (True, bias), (True, None)):
+        gu = [torch.zeros((n, N), dtype=torch.bfloat16, device="cuda") if swiglu else None for n in (S, S + 1801)]
+        got = g.grouped_mxfp4_gemm(x[:S], small, tn, ts, N, K, S, bias=b, swiglu=swiglu, gate_up=gu[0])
+        ref = g.grouped_mxfp4_gemm(x, large, tn, ts, N, K, S + 1801, bias=b, swiglu=swiglu, gate_up=gu[1])
+        assert torch.equal(got.view(torch.int16), ref[:S].view(torch.int16))
+        if swiglu:
+            assert torch.equal(gu[0].view(torch.int16), gu[1][:S].view(torch.int16))
+
+
+# The layer's products: rows gathered through the plan, the gate_up trace,
+# scale codes 0 and 255, with and without biases.  The first T tokens of a
+# larger forward (more than 1800 rows) take the other kernel: the same bits.
+@pytest.mark.parametrize("H,I", [(512, 576), (832, 704)])
+@pytest.mark.parametrize("T", [130, 450])
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("bias", [True, False])
+def test_mid_stream_layer(H, I, T, special, bias):
+    E, k, fill = 64, 4, 460
+    tiled = (*_random_tiled(E, 2 * I, H, special, 1), *_random_tiled(E, H, I, special, 2))
+    gen = torch.Generator(device="cuda").manual_seed(T)
+
+    def randn(*shape, scale=1.0):
+        return (scale * torch.randn(shape, device="cuda", generator=gen)).to(torch.bfloat16)
+
+    rw, rb = randn(E, H, scale=0.02), randn(E, scale=0.02)
+    b1, b2 = (randn(E, 2 * I, scale=0.5), randn(E, H, scale=0.5)) if bias else (None, None)
+    cfg = g.default_config(E, T + fill)
+    cfg.hidden_size, cfg.intermediate_size, cfg.top_k = H, I, k
+    layer = g.MoELayer().init(cfg, 0, rw, rb, b1, b2, tiled=tiled)
+    layer.set_trace_gate_up(True)
+    x, res = randn(T + fill, H), randn(T + fill, H)
+    # expert popularity by a power law, so that chunks of all heights occur
+    logp = -1.1 * torch.log(torch.arange(E, device="cuda") + 1.0)
+    noise = -torch.log(-torch.log(torch.rand((T + fill, E), device="cuda", generator=gen).clamp_(1e-6, 1 - 1e-6)))
+    idx = (logp + noise).topk(k, dim=1).indices.to(torch.int32).contiguous()
+    wts = torch.softmax(torch.randn((T + fill, k), device="cuda", generator=gen), dim=1).contiguous()
+
+    def stages(n):
+        out = layer.forward_routed(x[:n], idx[:n], wts[:n], residual=res[:n])
+        torch.cuda.synchronize()
+        tr, S = layer.trace(), n * k
+        gm = g.copy_device_to_tensor(tr.gather_map, S * 4, torch.int32)[:T * k].long()
+        rows = [g.copy_device_to_tensor(p, S * w * 2, torch.int16).view(S, w)[gm]
+                for p, w in ((tr.gate_up, 2 * I), (tr.act, I), (tr.expert_out, H))]
+        return [*rows, out[:T].view(torch.int16)]
+
+    for what, a, b in zip(("gate_up", "activations", "expert outputs", "out"), stages(T), stages(T + fill)):
+        assert torch.equal(a, b), what
+    layer.destroy()
+
+
 # What the grouped product refuses (an expert's nibbles of 2 GiB or more) it
 # refuses at every row count.  The buffers are real: nothing would be read out
 # of range if a call were taken.
