@@ -10,8 +10,8 @@
 //   expert_stream_kernel<!gated>  down: + bias, bf16 expert outputs
 //   combine8_kernel               out = bf16(sum_k w_k * y_k + residual)
 //
-// The stream kernel is persistent: at most two work-groups per CU (three up to
-// 8 slots) walk the (active expert, tile group, token chunk) steps of the
+// The stream kernel is persistent: at most two work-groups per CU (three for
+// small batches) walk the (active expert, tile group, token chunk) steps of the
 // routing plan's task records, so the weights stream without a gap between
 // steps (see expert_stream_kernel).
 //
@@ -133,7 +133,7 @@ struct StreamParams {
   const int32_t* perm_token;  // [S] token of each permuted slot (gate_up only)
   uint16_t* out;              // gate_up: SwiGLU activations [S][N/2]; down: expert outputs [S][N]
   uint16_t* gate_up;          // [S][N] bf16 trace or null (gate_up only)
-  int max_active;
+  int max_active, max_more;   // bounds of the active experts and of all chunks past their first
   float alpha, limit;
   TiledGeom g;                // [N, K] geometry
 };
@@ -164,7 +164,7 @@ struct Step {
 // wave's loads never stop between steps; loads for a step that does not
 // exist read a fixed valid location (static wait counts, no stray traffic).
 template <int BPP, int R, int TC, int D, bool kGated>
-__global__ __launch_bounds__(kTileRows * kMaxParts) __attribute__((amdgpu_waves_per_eu(R == 1 ? 5 : 4)))
+__global__ __launch_bounds__(kTileRows * kMaxParts) __attribute__((amdgpu_waves_per_eu(R == 1 && BPP != 0 ? 5 : 4)))
 void expert_stream_kernel(StreamParams a) {
   constexpr int PK = PartLen<BPP, R>::kValue;
   static_assert(TC * R * kTileRows <= TC * PK, "part sums fit the staged rows");
@@ -217,6 +217,10 @@ void expert_stream_kernel(StreamParams a) {
 #pragma unroll
       for (int i = 0; i < kRec; ++i) {
         const int r = lane + i * kWave;
+        if (i * kWave >= a.max_active) {  // no records: nothing to scan
+          sm.more[r] = base;
+          continue;
+        }
         sm.hdr[r] = make_int2(hv[i].x < 0 ? -1 : (hv[i].x | (hv[i].z << 8)), hv[i].y);
         int n = hv[i].x < 0 ? 0 : (hv[i].z - 1) / TC;
 #pragma unroll
@@ -230,6 +234,7 @@ void expert_stream_kernel(StreamParams a) {
     }
     __syncthreads();
   };
+  const int nsteps = nfirst + a.max_more * ntp;  // the list ends here at the latest
   auto step_of = [&](int q) -> Step {
     Step n;
     n.q = q;
@@ -237,6 +242,9 @@ void expert_stream_kernel(StreamParams a) {
     if (q < nfirst) {
       n.j = q / ntp;
       n.tp = q - n.j * ntp;
+    } else if (q >= nsteps) {
+      n.j = nact;
+      n.tp = 0;
     } else {
       const int x = (q - nfirst) / ntp;  // the x-th further chunk
       n.tp = q - nfirst - x * ntp;
@@ -625,14 +633,24 @@ __global__ void pack_mscale_kernel(const uint8_t* __restrict__ src, int N, int n
 }  // namespace
 
 // Launch shapes.  Two rows on each lane halve the LDS activation traffic per
-// fmaf and a chunk of four tokens the weight decode; a batch of up to 8 routed
-// slots (2 tokens at top-4) has at most a few steps per work-group and waits
-// for latency, so it takes one row per lane (twice the steps) and three
-// work-groups per CU instead of two.  A 20B layer of 1 / 2 / 4 / 8 tokens:
-// one row 35 / 47 / 68 / 104 us, two rows 41 / 52 / 64 / 87 us.  The grid
-// never exceeds the steps a launch can have (first chunks: max_active x tile
-// groups; further ones: at most one per TC slots) nor what stays resident on
-// the device.
+// fmaf and a chunk of four tokens the weight decode; a batch that has at most a
+// few steps per work-group waits for latency and takes one row per lane (twice
+// the steps) and three work-groups per CU instead of two.  That is: up to 8
+// routed slots (2 tokens at top-4; a 20B layer of 1 / 2 / 4 / 8 tokens: one row
+// 35 / 47 / 68 / 104 us, two rows 41 / 52 / 64 / 87 us), and every batch whose
+// steps are all resident at once (16 experts of 512 x 512, top-2, 5 tokens:
+// 31.5 us with two rows, 22.8 with one).
+//
+// A part of any number of blocks other than 15 and 1 goes through the loop of
+// 16 guarded blocks: one row per lane then holds the whole part in flight and
+// takes chunks of two tokens, since a short batch runs the unrolled code about
+// once and waits for its instructions (64 experts, top-8, 1024 x 768, 1 token:
+// 29.3 us with four blocks and four tokens, 25 so), and it stays ahead of two
+// rows up to 64 slots (2048 x 2048, 5 tokens: 140 against 87 us).
+//
+// The grid never exceeds the steps a launch can have (first chunks: max_active
+// x tile groups; further ones: at most one per TC slots) nor what stays
+// resident on the device.
 template <int BPP, int R, int TC, int D, bool kGated>
 static void launch_stream_t(const ExpertArgs& a, const TiledGeom& g, hipStream_t s) {
   StreamParams p{};
@@ -646,11 +664,12 @@ static void launch_stream_t(const ExpertArgs& a, const TiledGeom& g, hipStream_t
   p.out = kGated ? a.act : a.y;
   p.gate_up = kGated ? a.gate_up : nullptr;
   p.max_active = a.max_active;
+  p.max_more = a.T * a.k / TC;
   p.alpha = a.alpha;
   p.limit = a.limit;
   p.g = g;
   const int ntp = (g.N / kTileRows + R - 1) / R;
-  const int items = (a.max_active + a.T * a.k / TC) * ntp;
+  const int items = (a.max_active + p.max_more) * ntp;
   const int resident = 256 * (R == 1 ? 3 : 2);
   const int grid = items < resident ? items : resident;
   gx_launch(expert_stream_kernel<BPP, R, TC, D, kGated>, dim3(grid), dim3(kTileRows * g.parts), 0, s, a.timer, p);
@@ -659,7 +678,10 @@ static void launch_stream_t(const ExpertArgs& a, const TiledGeom& g, hipStream_t
 template <int BPP, bool kGated>
 static void launch_stream_b(const ExpertArgs& a, const TiledGeom& g, hipStream_t s) {
   constexpr int D = BPP == 15 ? 3 : BPP == 1 ? 1 : 4;
-  if (a.T * a.k <= 8) launch_stream_t<BPP, 1, 4, D, kGated>(a, g, s);
+  constexpr int D1 = BPP ? D : kMaxBpp, TC1 = BPP == 15 ? 4 : 2;
+  const int S = a.T * a.k, resident = 256 * 3;
+  const long steps = static_cast<long>(a.max_active + S / TC1) * (g.N / kTileRows);
+  if (S <= (BPP ? 8 : 64) || steps <= resident) launch_stream_t<BPP, 1, TC1, D1, kGated>(a, g, s);
   else launch_stream_t<BPP, 2, 4, D, kGated>(a, g, s);
 }
 

@@ -89,9 +89,9 @@ def test_layer_plan(E, k, T):
 
 
 # exact decode under skewed routing, token for token the bits of a batch of
-# one: K-parts of an odd and an even number of blocks, one to six of them; one row per lane (up to 8
-# slots) or two; more and fewer first chunks than work-groups, experts from
-# one token to all of them, more records than one wave holds
+# one: K-parts of an odd and an even number of blocks, one to six of them; one
+# row per lane or two; experts from one token to all of them, more records than
+# one wave holds
 @pytest.mark.parametrize("E,k,H,I", [(1, 1, 128, 64), (30, 4, 448, 192), (200, 4, 128, 64), (8, 2, 2880, 960)])
 @pytest.mark.parametrize("T", [1, 2, 3, 17, 64, 150])
 def test_exact_steps(E, k, H, I, T):
@@ -115,6 +115,26 @@ def test_exact_steps(E, k, H, I, T):
         one = layer.forward_routed(dx[i:i + 1].contiguous(), idx[i:i + 1].contiguous(), wts[i:i + 1].contiguous(),
                                    residual=dr[i:i + 1].contiguous())
         assert np.array_equal(_bits(one)[0], got[i]), i
+    layer.destroy()
+
+
+# The same against the oracle: one row per lane (up to 64 slots, or all steps
+# resident) and two; more first chunks than work-groups in both (64 experts, 8
+# and 40 tokens at top-8); parts of 16, 8, 4, 3 and 2 blocks
+@pytest.mark.parametrize("E,k,H,I", [(64, 8, 1024, 768), (6, 2, 2048, 576), (12, 4, 640, 384)])
+@pytest.mark.parametrize("T", [1, 3, 8, 9, 40])
+def test_exact_steps_oracle(E, k, H, I, T):
+    w = moe_data.make_layer(5, E, H, I, bias="random")
+    x, res = moe_data.make_tokens(T, T, H)
+    idx, wts = moe_data.zipf_routing(T, T, E, k, s=0.2)
+    cfg = g.default_config(E, T, decode_exact=True, prefill_min_tokens=0)
+    cfg.hidden_size, cfg.intermediate_size, cfg.top_k = H, I, k
+    t = {n: _dev(v) for n, v in w.items()}
+    layer = g.MoELayer().init(cfg, 0, t["router_w"], t["router_b"], t["w1_bias"], t["w2_bias"],
+                              mlp1=([t["w1_packed"][e] for e in range(E)], [t["w1_scales"][e] for e in range(E)]),
+                              mlp2=([t["w2_packed"][e] for e in range(E)], [t["w2_scales"][e] for e in range(E)]))
+    got = _bits(layer.forward_routed(_dev(x), _dev(idx), _dev(wts), residual=_dev(res)))
+    assert np.array_equal(got, orc.moe_forward_routed(w, x, res, idx, wts, E, k, H, I))
     layer.destroy()
 
 
