@@ -35,10 +35,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // come through the scalar cache into scalar registers, a block of a row in one
 // 64-byte load, and each fmaf takes one as its scalar operand (as LDS
 // broadcasts, 16 bytes per four fmaf, they ran at the LDS rate).  The block
-// loop is kept rolled: unrolled over the part it waits for instructions.
+// loop is kept rolled: unrolled over the part it waits for instructions.  Rows
+// that start between two dwords (kShift; x then points to element 1, so that
+// every part of a scalar load's address is on four bytes) take the 30 elements
+// of a block that whole dwords hold the same way and the two others from one
+// load per lane ahead of the loop (element by element through vector loads,
+// each of which waits for the weights in flight: N = 201088, M = 1: 605 us).
 // Measured, N = 5760, K = 2880, M = 1 / 5 / 16 / 64: 20.5 / 48 / 70 / 115 us
 // before, 8.1 / 13.1 / 21 / 62 now.
-template <int TC, bool kAligned>
+template <int TC, bool kShift>
 __global__ __launch_bounds__(kTileRows * kMaxParts) void dense_gemv_kernel(
     const uint16_t* __restrict__ x, int M, const uint8_t* __restrict__ wn, const uint8_t* __restrict__ ws,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, TiledGeom g) {
@@ -54,7 +59,7 @@ __global__ __launch_bounds__(kTileRows * kMaxParts) void dense_gemv_kernel(
   const uint8_t* sc = ws + (static_cast<size_t>(tile) * g.parts + p) * kTileRows * g.spad +
                       static_cast<size_t>(lane) * g.spad;
   uint32_t codes[4];  // the part's scale codes, at most 16
-  if (kAligned) {
+  if ((reinterpret_cast<uintptr_t>(ws) & 3u) == 0) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) codes[q] = reinterpret_cast<const uint32_t*>(sc)[min(q, (g.spad >> 2) - 1)];
   } else {
@@ -71,6 +76,16 @@ __global__ __launch_bounds__(kTileRows * kMaxParts) void dense_gemv_kernel(
   const uint16_t* xr[TC];  // rows past M: the last row, their sums are not stored
 #pragma unroll
   for (int m = 0; m < TC; ++m) xr[m] = x + static_cast<size_t>(m0 + min(m, mc - 1)) * K + p * bpp * 32;
+  // kShift: lane 2 i holds each row's first element of block i, lane 2 i + 1
+  // its last (the block's other 30 lie in whole dwords)
+  float edge[kShift ? TC : 1];
+  if constexpr (kShift) {
+#pragma unroll
+    for (int m = 0; m < TC; ++m) edge[m] = bf16_to_f32(xr[m][32 * min(lane >> 1, bpp - 1) + 31 * (lane & 1) - 1]);
+  }
+  auto edge_of = [&](int m, int l) -> float {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(edge[m]), l));
+  };
   float acc[TC];
 #pragma unroll
   for (int m = 0; m < TC; ++m) acc[m] = 0.0f;
@@ -92,25 +107,29 @@ __global__ __launch_bounds__(kTileRows * kMaxParts) void dense_gemv_kernel(
           for (int c = 0; c < 32; ++c) wf[c] = sp ? wf[c] * scale : wf[c];
         }
         wv[u] = src[static_cast<size_t>(min(i + kD, bpp - 1)) * 64];
-        if constexpr (kAligned) {
-          uint32_t xv[TC][16];
+        // the rows' chains side by side, a dword of two elements at a time
+        constexpr int kDw = kShift ? 15 : 16;
+        uint32_t xv[TC][kDw];
+#pragma unroll
+        for (int m = 0; m < TC; ++m)
+#pragma unroll
+          for (int c = 0; c < kDw; ++c) xv[m][c] = reinterpret_cast<const uint32_t*>(xr[m] + 32 * i)[c];
+        if constexpr (kShift) {
+#pragma unroll
+          for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(edge_of(m, 2 * i), wf[0], acc[m]);
+        }
+#pragma unroll
+        for (int c = 0; c < kDw; ++c) {
+          constexpr int k0 = kShift ? 1 : 0;
+#pragma unroll
+          for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(__uint_as_float(xv[m][c] << 16), wf[2 * c + k0], acc[m]);
 #pragma unroll
           for (int m = 0; m < TC; ++m)
+            acc[m] = __builtin_fmaf(__uint_as_float(xv[m][c] & 0xffff0000u), wf[2 * c + 1 + k0], acc[m]);
+        }
+        if constexpr (kShift) {
 #pragma unroll
-            for (int c = 0; c < 16; ++c) xv[m][c] = reinterpret_cast<const uint32_t*>(xr[m] + 32 * i)[c];
-#pragma unroll
-          for (int c = 0; c < 16; ++c) {  // the rows' chains side by side
-#pragma unroll
-            for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(__uint_as_float(xv[m][c] << 16), wf[2 * c], acc[m]);
-#pragma unroll
-            for (int m = 0; m < TC; ++m)
-              acc[m] = __builtin_fmaf(__uint_as_float(xv[m][c] & 0xffff0000u), wf[2 * c + 1], acc[m]);
-          }
-        } else {
-#pragma unroll
-          for (int c = 0; c < 32; ++c)
-#pragma unroll
-            for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(bf16_to_f32(xr[m][32 * i + c]), wf[c], acc[m]);
+          for (int m = 0; m < TC; ++m) acc[m] = __builtin_fmaf(edge_of(m, 2 * i + 1), wf[31], acc[m]);
         }
       }
     }
@@ -310,15 +329,14 @@ hipError_t launch_dense_gemv(const uint16_t* x, int M, const uint8_t* wn, const 
   const int tiles = N / kTileRows;
   const long groups = static_cast<long>(tiles) * M;
   const int tc = groups <= 1024 ? 1 : groups <= 2560 ? 2 : 4;
-  // x is only 2-byte aligned by contract, the scales not at all
-  const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(ws)) & 3u) == 0;
+  const bool shift = (reinterpret_cast<uintptr_t>(x) & 2u) != 0;  // x is only 2-byte aligned by contract
 #define GX_GEMV(TC_, A_)                                                                                            \
   hipLaunchKernelGGL((dense_gemv_kernel<TC_, A_>), dim3(tiles, (M + TC_ - 1) / TC_), dim3(kTileRows* g.parts), 0, s, \
-                     x, M, wn, ws, bias, y, g)
-#define GX_GEMV_L(TC_)               \
-  do {                               \
-    if (aligned) GX_GEMV(TC_, true); \
-    else GX_GEMV(TC_, false);        \
+                     x + (A_ ? 1 : 0), M, wn, ws, bias, y, g)
+#define GX_GEMV_L(TC_)             \
+  do {                             \
+    if (shift) GX_GEMV(TC_, true); \
+    else GX_GEMV(TC_, false);      \
   } while (0)
   if (tc == 1) GX_GEMV_L(1);
   else if (tc == 2) GX_GEMV_L(2);
