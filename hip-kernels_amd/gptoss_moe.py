@@ -765,8 +765,8 @@ def permute_plan(idx, num_experts: int, stream=None):
     counts = torch.empty(num_experts, dtype=torch.int32, device=dev)
     offsets = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
     gmap = torch.empty(S, dtype=torch.int32, device=dev)
-    # the entries a plan leaves unwritten read -1; one fill for both
-    ptok, active = torch.full((S + num_experts,), -1, dtype=torch.int32, device=dev).split((S, num_experts))
+    ptok = torch.full((S,), -1, dtype=torch.int32, device=dev)
+    active = torch.full((num_experts,), -1, dtype=torch.int32, device=dev)
     n_active = torch.empty(1, dtype=torch.int32, device=dev)
     check(_lib.gptoss_moe_permute_plan(_ptr(idx), T, k, num_experts, _ptr(counts), _ptr(offsets), _ptr(gmap),
                                        _ptr(ptok), _ptr(active), _ptr(n_active), _stream(stream)))

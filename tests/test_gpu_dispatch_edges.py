@@ -88,6 +88,19 @@ def test_layer_plan(E, k, T):
     layer.destroy()
 
 
+# a plan's tensors are a caller's to write, resize and index with: they share
+# neither memory nor a version counter
+def test_plan_tensors_are_separate():
+    idx = torch.randint(0, 30, (7, 4), dtype=torch.int32, device="cuda")
+    p = g.permute_plan(idx, 30)
+    assert len({t.untyped_storage().data_ptr() for t in p.values()}) == len(p)
+    x = torch.randn((7, 8), device="cuda", requires_grad=True)
+    rows = x[p["perm_token"]]
+    p["active"].fill_(0)
+    rows.sum().backward()
+    assert torch.equal(x.grad, torch.full_like(x, 4.0))
+
+
 # exact decode under skewed routing, token for token the bits of a batch of
 # one: K-parts of an odd and an even number of blocks, one to six of them; one
 # row per lane or two; experts from one token to all of them, more records than
