@@ -5,6 +5,7 @@ include/cuda_utils.h:17-35).  None of these calls reaches a kernel launch."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -29,6 +30,16 @@ def test_exports_every_declared_symbol(g):
     assert len(names) >= 20
     missing = [n for n in names if not hasattr(g.lib, n)]
     assert not missing, missing
+
+
+@pytest.mark.parametrize("build", ["hip-kernels_amd", os.path.join("tests", "sanitize")])
+def test_builds_link_every_source(build):
+    """The library and its sanitizer build both take every HIP source: one
+    left out is an undefined symbol only when the library is opened."""
+    r = subprocess.run(["make", "-C", os.path.join(ROOT, build), "-pn", "all"], capture_output=True, text=True)
+    listed = re.search(r"^SOURCES :?= (.*)$", r.stdout, flags=re.M)[1].split()
+    csrc = os.path.join(ROOT, "hip-kernels_amd", "csrc")
+    assert sorted(listed) == sorted(f[:-4] for f in os.listdir(csrc) if f.endswith(".hip"))
 
 
 def test_abi_version_and_defaults(g):
