@@ -47,7 +47,8 @@ constexpr int kMidWaves = 4;              // waves per work-group, a 64-row weig
 constexpr int kMidPerCU = 2;              // work-groups per CU
 constexpr int kMidFrags = 4;              // 16-row token fragments per chunk
 constexpr int kMidRows = 16 * kMidFrags;  // rows per chunk
-constexpr int kMidChunks = 360;           // chunk table entries (LDS)
+constexpr int kMidMaxRows = 1800;         // rows of a call (the rule by size, below)
+constexpr int kMidChunks = kMaxExperts + kMidMaxRows / kMidRows;  // chunk table entries (LDS): all a call can have
 constexpr int kBufWord3 = 0x00020000;     // raw buffer, dword data (gfx9 descriptor word 3)
 constexpr int kNT = 2;                    // buffer load cache policy: nontemporal (streamed once)
 
@@ -95,6 +96,10 @@ __global__ __launch_bounds__(kMidWaves * kWave, kMidPerCU) void mid_stream_kerne
   __shared__ uint2 bs[kMidWaves][kTileRows / 4 + 1];
   __shared__ int2 tab[kMidChunks];                // chunks: {expert | rows << 8, first permuted row}
   __shared__ int tab_n, tail_item;
+
+  static_assert((sizeof(xs) + sizeof(scs) + sizeof(bs) + sizeof(tab) + sizeof(tab_n) + sizeof(tail_item)) * kMidPerCU <=
+                    160 * 1024,
+                "two work-groups per CU");
 
   const TiledGeom& g = a.g;
   const int lane = threadIdx.x & 63;
@@ -444,14 +449,14 @@ hipError_t launch_mid_t(const MidParams& p, int grid, hipStream_t s, const Kerne
 // 186 / 240.  So: up to 1800 rows, and up to 50 on average per expert.
 bool mid_stream_pays(const GroupedArgs& a) {
   const int active = a.E < a.rows ? a.E : a.rows;
-  return a.rows <= 1800 && a.rows <= 50 * active;
+  return a.rows <= kMidMaxRows && a.rows <= 50 * active;
 }
 
 bool mid_stream_supported(const GroupedArgs& a) {
   if (!grouped_supported(a.N, a.K, a.E) || a.x_rows <= 0 || a.num_cus <= 0 || a.xq != nullptr) return false;
   const TiledGeom g = tiled_geom(a.N, a.K);
   if (g.nb <= 9) return false;  // one phase: a next item's rows would not be known in time
-  if (a.E + a.rows / kMidRows > kMidChunks) return false;
+  if (a.rows > kMidMaxRows) return false;  // the chunk table
   constexpr size_t kMaxBuf = 0xffff0000u;  // 32-bit buffer offsets, with room for the lanes' terms
   const size_t S = static_cast<size_t>(a.rows);
   return g.nib_bytes * a.E <= kMaxBuf && g.scale_bytes * a.E <= kMaxBuf && S * 4 <= kMaxBuf &&

@@ -162,6 +162,21 @@ def test_mid_stream_many_items(K, special, routing):
             assert torch.equal(gu[0].view(torch.int16), gu[1][:S].view(torch.int16))
 
 
+# The most chunks a call can have: 1800 rows, 255 of 256 experts with one each
+def test_mid_stream_most_chunks():
+    E, N, K, S = 256, 64, 320, 1800
+    tn, ts = _random_tiled(E, N, K, False, 9)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn((S + 128, K), device="cuda", generator=gen).to(torch.bfloat16)
+    for big in (0, 100, 255):
+        counts = np.ones(E, dtype=np.int64)
+        counts[big] = S - (E - 1)
+        offs = np.concatenate([[0], np.cumsum(counts)])
+        got = g.grouped_mxfp4_gemm(x[:S], _dev(offs.astype(np.int32)), tn, ts, N, K, S)
+        ref = g.grouped_mxfp4_gemm(x, _dev(offs.astype(np.int32)), tn, ts, N, K, S + 128)
+        assert torch.equal(got.view(torch.int16), ref[:S].view(torch.int16))
+
+
 # The layer's products: rows gathered through the plan, the gate_up trace,
 # scale codes 0 and 255, with and without biases.  The first T tokens of a
 # larger forward (more than 1800 rows) take the other kernel: the same bits.
