@@ -469,12 +469,13 @@ def test_gptoss120b_prefill_block_scaled_error(gpu, orc, torch_mod, zipf120, mod
     exact.set_trace_gate_up(False)
 
 
-@pytest.mark.parametrize("T", [300, 2000])
+@pytest.mark.parametrize("T", [300, 1024, 1025, 2000])
 def test_layer_plan_many_slots(gpu, orc, torch_mod, T):
-    """The layer's plan for more than 1024 slots (three launches over the
-    device: per-chunk counts, scan, placement) against the oracle's counting
-    sort, array by array: counts, offsets, stable gather map, permuted tokens
-    and the active list, with dropped slots (-1 and >= E)."""
+    """The layer's plan for up to 4096 slots (one work-group) and more (three
+    launches over the device: per-chunk counts, scan, placement; 1025 tokens:
+    a last chunk of four slots) against the oracle's counting sort, array by
+    array: counts, offsets, stable gather map, permuted tokens and the active
+    list, with dropped slots (-1 and >= E)."""
     torch = torch_mod
     E, k, H, I = 128, 4, 128, 128
     w = moe_data.make_layer(70 + T, E, H, I)
