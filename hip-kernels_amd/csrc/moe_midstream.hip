@@ -28,13 +28,14 @@
 // same instruction and order as grouped_mfma_kernel, so both give the same
 // bits.
 //
-// Measured (GPT-OSS-120B layer, HIP events per launch, against
-// grouped_mfma_kernel; uniform routing): 200 tokens gate_up 192 against 227 us
-// (5.9 TB/s of weights), down 96 against 119; 512 tokens 212 against 249 and
-// 111 against 129.  What bounds it: at 200 tokens a copy of the kernel without
-// products and decode takes the same 193 us, one without weight loads 155, so
-// it is the stream (72 KiB in flight per CU) and the phase barriers; from about
-// 1000 tokens the epilogue (40 us of 253) and the products.
+// Measured (GPT-OSS-120B layer, kernel trace, 200 tokens, uniform routing):
+// gate_up 190 us against 227 in grouped_mfma_kernel, down 98 against 119; it
+// reads 1.01 of the touched weights' bytes, at 6.0 TB/s.  What bounds it: a copy
+// of the kernel without products and decode takes 184 us where this takes 200
+// (450 tokens: 203 of 214), one without weight loads 165 (172), so neither the
+// stream nor the rest hides wholly behind the other.  Waves issue for 0.49 of
+// their cycles, wait to issue for 0.33 and on counters for 0.18; the matrix
+// cores are busy for 0.3.
 #include "moe_device.h"
 #include "moe_kernels.h"
 
@@ -440,13 +441,21 @@ hipError_t launch_mid_t(const MidParams& p, int grid, hipStream_t s, const Kerne
 
 }  // namespace
 
-// The rule by size.  Measured, GPT-OSS shapes, layer us (old / this kernel),
-// uniform and Zipf(1.1) routing: 128 experts, 512 rows 356 / 296 and 277 / 261;
-// 800 rows 357 / 303 and 320 / 281; 2048 rows 396 / 342 and 392 / 393; 4004 rows
-// 443 / 400 but 461 / 506: a few experts then hold most rows, and a 64-row
-// chunk costs their products more than a 128-row tile does.  32 experts, 800
-// rows 139 / 120 and 169 / 132; 1600 rows 163 / 155 and 191 / 170; 2400 rows
-// 186 / 240.  So: up to 1800 rows, and up to 50 on average per expert.
+// The rule by size.  Measured, GPT-OSS shapes, layer us (grouped_mfma_kernel /
+// this kernel), uniform and Zipf(1.1) routing: 128 experts, 512 rows 356 / 296
+// and 277 / 261; 800 rows 357 / 303 and 320 / 281; 2048 rows 396 / 342 and 392 /
+// 393; 4004 rows 443 / 400 but 461 / 506: a few experts then hold most rows, and
+// a 64-row chunk costs their products more than a 128-row tile does.  32
+// experts, 800 rows 139 / 120 and 169 / 132; 1600 rows 163 / 155 and 191 / 170;
+// 2400 rows 186 / 240.  So: up to 1800 rows, and up to 50 on average per expert.
+//
+// Over what the rule admits, one product at a time (1 to 256 experts, eight
+// shapes from 64 x 320 to 5760 x 2880, 8 to 1800 rows, uniform and Zipf(1.1)
+// routing and all rows on four experts or one; 2184 points), this kernel takes
+// 0.75 of the other's time on average and at most 1.03, but for down products
+// of 64 experts, 2880 x 2880, 800 to 1600 rows, where single Zipf draws reach
+// 1.08 (0.97 over eight draws).  Closest: 1800 rows on one expert, gate_up of
+// the 120B layer, 75.5 / 74.5 us.
 bool mid_stream_pays(const GroupedArgs& a) {
   const int active = a.E < a.rows ? a.E : a.rows;
   return a.rows <= kMidMaxRows && a.rows <= 50 * active;

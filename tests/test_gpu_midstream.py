@@ -1,9 +1,9 @@
 """The grouped product for a few tokens per expert (moe_midstream.hip), which
 launch_grouped_mxfp4 takes up to 1800 rows and 50 rows per expert.  Its chain
 of matrix-core products is grouped_mfma_kernel's, so the same rows give the
-same bits in a larger call that takes that kernel: every case appends filler
-rows on one more expert until the call leaves the range, and compares the
-original rows.  Against fp64 the result is one bf16 rounding away."""
+same bits in a larger call that takes that kernel: the cases append filler rows
+until the call leaves the range, and compare the original rows.  Against fp64
+the result is one bf16 rounding away."""
 import numpy as np
 import pytest
 import torch
