@@ -48,6 +48,23 @@ def test_gemv_rows(N, K, M, shift):
     assert np.array_equal(y[~nan], ref[~nan])
 
 
+# scales off a dword (no alignment is asked of them), with x on and off one
+@pytest.mark.parametrize("N,K", [(64, 96), (128, 960), (64, 2048)])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_gemv_scales_unaligned(N, K, off):
+    rng = np.random.default_rng([N, K])
+    M = 5
+    x = moe_data.bf16(rng.normal(0, 1, (M, K)))
+    packed = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    scales = rng.integers(119, 124, (N, K // 32), dtype=np.uint8)
+    nib, sc = g.pack_tiled(_dev(packed), _dev(scales), N, K)
+    moved = torch.zeros(sc.numel() + 8, dtype=torch.uint8, device="cuda")[off:off + sc.numel()]
+    moved.copy_(sc.flatten())
+    ref = orc.mxfp4_gemv(x, packed, scales, None, N, K)
+    for shift in (0, 1):
+        assert np.array_equal(_bits(g.mxfp4_gemv(_shifted(x, shift), nib, moved, None, N, K)), ref)
+
+
 # top-k and plan in one launch up to 64 tokens, plan in one work-group up to
 # 4096 slots, over the chip above
 @pytest.mark.parametrize("E,k", [(30, 4), (64, 8), (128, 4)])
