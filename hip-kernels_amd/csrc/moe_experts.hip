@@ -223,13 +223,15 @@ void expert_stream_kernel(StreamParams a) {
         }
         sm.hdr[r] = make_int2(hv[i].x < 0 ? -1 : (hv[i].x | (hv[i].z << 8)), hv[i].y);
         int n = hv[i].x < 0 ? 0 : (hv[i].z - 1) / TC;
+        if (__ballot(n > 0) != 0ull) {
 #pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-          const int u = __shfl_up(n, d, kWave);
-          n += lane >= d ? u : 0;
+          for (int d = 1; d < kWave; d <<= 1) {
+            const int u = __shfl_up(n, d, kWave);
+            n += lane >= d ? u : 0;
+          }
         }
         sm.more[r] = base + n;
-        base += __shfl(n, kWave - 1, kWave);
+        base += __builtin_amdgcn_readlane(n, kWave - 1);
       }
     }
     __syncthreads();
@@ -646,7 +648,9 @@ __global__ void pack_mscale_kernel(const uint8_t* __restrict__ src, int N, int n
 // takes chunks of two tokens, since a short batch runs the unrolled code about
 // once and waits for its instructions (64 experts, top-8, 1024 x 768, 1 token:
 // 29.3 us with four blocks and four tokens, 25 so), and it stays ahead of two
-// rows up to 64 slots (2048 x 2048, 5 tokens: 140 against 87 us).
+// rows up to 64 slots (2048 x 2048, 5 tokens: 140 against 87 us) while there are
+// as many experts as slots, so that most hold one chunk (24 experts of 1536 x
+// 1536, top-4, 8 tokens: two rows 53.8 us, one 55.9).
 //
 // The grid never exceeds the steps a launch can have (first chunks: max_active
 // x tile groups; further ones: at most one per TC slots) nor what stays
@@ -681,7 +685,8 @@ static void launch_stream_b(const ExpertArgs& a, const TiledGeom& g, hipStream_t
   constexpr int D1 = BPP ? D : kMaxBpp, TC1 = BPP == 15 ? 4 : 2;
   const int S = a.T * a.k, resident = 256 * 3;
   const long steps = static_cast<long>(a.max_active + S / TC1) * (g.N / kTileRows);
-  if (S <= (BPP ? 8 : 64) || steps <= resident) launch_stream_t<BPP, 1, TC1, D1, kGated>(a, g, s);
+  if (S <= 8 || steps <= resident || (BPP == 0 && S <= 64 && S <= a.E))
+    launch_stream_t<BPP, 1, TC1, D1, kGated>(a, g, s);
   else launch_stream_t<BPP, 2, 4, D, kGated>(a, g, s);
 }
 

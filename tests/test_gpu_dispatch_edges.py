@@ -148,7 +148,7 @@ def test_exact_steps(E, k, H, I, T):
     layer.destroy()
 
 
-# The same against the oracle: one row per lane (up to 64 slots, or all steps
+# The same against the oracle: one row per lane (few slots, or all steps
 # resident) and two; more first chunks than work-groups in both (64 experts, 8
 # and 40 tokens at top-8); parts of 16, 8, 4, 3 and 2 blocks
 @pytest.mark.parametrize("E,k,H,I", [(64, 8, 1024, 768), (6, 2, 2048, 576), (12, 4, 640, 384)])
